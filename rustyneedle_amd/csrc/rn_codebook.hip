@@ -12,7 +12,7 @@
 //   plane_input / NaturalInput::new per-group input codes (matrix.rs:205-214,
 //     neon.rs:63-106, panel.rs:52-66), PanelMatrix::tile (panel.rs:153-197,
 //     2-bit) and row_dot_two_bit / row_dot_four_bit (neon.rs:126-183, 4-bit
-//     and ternary crumbs)                                    -> cb_product_kernel
+//     and ternary crumbs)             -> cb_product_kernel, cb_tile_kernel (batches)
 //   QuantisedMatrix::dequantise_row (matrix.rs:140-153)      -> cb_dequantise_kernel
 //
 // Product arithmetic (bit-exact with the reference order):
@@ -34,6 +34,8 @@
 // {k, 4+k, 8+k, 12+k}; the codes of each run of 16 elements are stored as the
 // 4x4 byte transpose. For 4-bit indices a dword holds 8 elements and
 // (dword >> 4k) & 0x0f0f0f0f selects {k, 2+k, 4+k, 6+k}.
+#include <type_traits>
+
 #include "rn_device.hpp"
 #include "rn_internal.hpp"
 
@@ -104,17 +106,18 @@ __device__ __forceinline__ int4 plane_pack(const int (&c)[16]) {
                          b4(c[9], c[11], c[13], c[15]));
 }
 
-// The int8 levels of four indices (one per byte of sel, 0..3 or 0..15).
+// The int8 levels of four indices (one per byte of sel, 0..3 or 0..15; 4-bit: in
+// the low nibble, the high one is not looked at).
 template <int BITS>
 __device__ __forceinline__ int decode4(uint32_t sel, const uint32_t (&lut)[4]) {
     if constexpr (BITS == 2) {
         return (int)__builtin_amdgcn_perm(0u, lut[0], sel);
     } else {
+        // entries 0..7 and 8..15 of each byte's low three bits, then bit 3 picks the byte of one or the other
         const uint32_t s7 = sel & 0x07070707u;
         const uint32_t lo = __builtin_amdgcn_perm(lut[1], lut[0], s7);
         const uint32_t hi = __builtin_amdgcn_perm(lut[3], lut[2], s7);
-        const uint32_t m = ((sel >> 3) & 0x01010101u) * 0xffu;
-        return (int)((hi & m) | (lo & ~m));
+        return (int)__builtin_amdgcn_perm(hi, lo, ((sel >> 1) & 0x04040404u) | 0x03020100u);
     }
 }
 
@@ -179,7 +182,7 @@ __global__ __launch_bounds__(1024) void cb_dequantise_kernel(CodebookParams p, i
             if (16 * u + i < p.columns) out[16 * u + i] = v[i];
 }
 
-// The row products of T tokens at a time (token tile blockIdx.y). A block of
+// The row products of one token (blockIdx.y). A block of
 // four waves shares one prologue; each wave owns R = p.rows_per_block rows of a
 // row group of 4R rows, and the block runs p.iters consecutive row groups so
 // that a wide input is quantised once for many rows.
@@ -194,10 +197,9 @@ __global__ __launch_bounds__(1024) void cb_dequantise_kernel(CodebookParams p, i
 //   3. Per row group: decoded dwords meet code dwords in v_dot4 and the chunks
 //      of one group join across their lanes (DPP) into the wave's acc_s; the
 //      next row group's loads are issued before this one's epilogue;
-//   4. one lane per (token, row): the sequential group epilogue.
-template <int BITS, int GROUP, int FORM, int NL, int T>
-__device__ __forceinline__ void cb_product_body(const CodebookParams& p, const float* x, int count, float* y,
-                                                int32_t* acc_out) {
+//   4. one lane per row: the sequential group epilogue.
+template <int BITS, int GROUP, int FORM, int NL>
+__device__ __forceinline__ void cb_product_body(const CodebookParams& p, const float* x, float* y, int32_t* acc_out) {
     constexpr int IB = BITS == 5 ? 2 : BITS;        // index bits (ternary crumbs are 2)
     constexpr int EPC = 128 / IB;                    // elements per 16-byte chunk
     constexpr int CPG = GROUP / EPC;                 // chunks per group
@@ -208,20 +210,17 @@ __device__ __forceinline__ void cb_product_body(const CodebookParams& p, const f
 
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int R = p.rows_per_block, CPR = p.cpr, G = p.padded / GROUP, runs = p.padded / 16;
-    const int BR = NW * R, t0 = blockIdx.y * T;
+    const int BR = NW * R;
+    x += (size_t)blockIdx.y * p.padded;
     uint16_t* nm_s = reinterpret_cast<uint16_t*>(lds);                                 // 12 KB of norms
-    int8_t* xq_s = reinterpret_cast<int8_t*>(lds + kNormWindow);                      // [T][padded]
-    int* acc_all = reinterpret_cast<int*>(lds + kNormWindow + (size_t)T * p.padded);  // [NW][T][R][G]
-    float* sx_s = reinterpret_cast<float*>(acc_all + (size_t)NW * T * R * G);         // [T][G]
-    int* acc_s = acc_all + (size_t)wv * T * R * G;
+    int8_t* xq_s = reinterpret_cast<int8_t*>(lds + kNormWindow);                      // [padded]
+    int* acc_all = reinterpret_cast<int*>(lds + kNormWindow + p.padded);               // [NW][R][G]
+    float* sx_s = reinterpret_cast<float*>(acc_all + (size_t)NW * R * G);              // [G]
+    int* acc_s = acc_all + (size_t)wv * R * G;
 
     // 1. requests
-    const int xruns = T * runs;  // flat (token, run) index of the tile
     auto load_run = [&](int f, float (&v)[16]) {
-        const int ff = min(f, xruns - 1);
-        const int t = ff / runs;
-        const float4* s = reinterpret_cast<const float4*>(x + (size_t)min(t0 + t, count - 1) * p.padded +
-                                                          16 * (ff - t * runs));
+        const float4* s = reinterpret_cast<const float4*>(x + 16 * min(f, runs - 1));
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const float4 q = s[i];
@@ -235,8 +234,8 @@ __device__ __forceinline__ void cb_product_body(const CodebookParams& p, const f
     load_run(tid, xv);
     // With DB, row groups alternate between two sets of weight registers and a
     // group's weights are requested before the previous group's decode;
-    // otherwise (wide rows, token tiles: no registers to spare) after it.
-    constexpr bool DB = NL == 8 && T == 1;
+    // otherwise (wide rows: no registers to spare) after it.
+    constexpr bool DB = NL == 8;
     v4i wa[NL], wb[DB ? NL : 1];
     v4i nv[3];  // native vectors stay in registers (arrays of int4 structs may not)
     auto group_row0 = [&](int it) -> int { return (blockIdx.x * p.iters + it) * BR; };
@@ -284,14 +283,13 @@ __device__ __forceinline__ void cb_product_body(const CodebookParams& p, const f
             for (int i = 0; i < 4; ++i) c[c4 + i] = code_of_quotient(q[i]);
             __builtin_amdgcn_sched_barrier(0);
         }
-        if (f < xruns) {
+        if (f < runs) {
             reinterpret_cast<int4*>(xq_s)[f] = plane_pack<IB>(c);
-            const int t = f / runs, u = f - t * runs;
-            if (u % RPG == 0) sx_s[t * G + u / RPG] = sx;
+            if (f % RPG == 0) sx_s[f / RPG] = sx;
         }
     };
     quantise_run(xv, tid);
-    for (int base = NT; base < xruns; base += NT) {  // wide inputs or many tokens
+    for (int base = NT; base < runs; base += NT) {  // wide inputs
         load_run(base + tid, xv);
         quantise_run(xv, base + tid);
     }
@@ -315,9 +313,7 @@ __device__ __forceinline__ void cb_product_body(const CodebookParams& p, const f
             const int idx = 64 * j + lane;
             const int rl = (int)(((float)idx + 0.5f) * p.inv_cpr);
             const int c = idx - rl * CPR;
-            int part[T];
-#pragma unroll
-            for (int t = 0; t < T; ++t) part[t] = 0;
+            int part = 0;
 #pragma unroll
             for (int d = 0; d < 4; ++d) {
                 const uint32_t wd = (uint32_t)w[j][d];
@@ -325,32 +321,18 @@ __device__ __forceinline__ void cb_product_body(const CodebookParams& p, const f
 #pragma unroll
                     for (int k = 0; k < 4; ++k) {
                         const int lv = decode4<2>((wd >> (2 * k)) & 0x03030303u, lut);
-#pragma unroll
-                        for (int t = 0; t < T; ++t) {
-                            const int a =
-                                *reinterpret_cast<const int*>(xq_s + (size_t)t * p.padded + 64 * c + 16 * d + 4 * k);
-                            part[t] = dot4(lv, a, part[t]);
-                        }
+                        part = dot4(lv, *reinterpret_cast<const int*>(xq_s + 64 * c + 16 * d + 4 * k), part);
                     }
                 } else {
 #pragma unroll
                     for (int k = 0; k < 2; ++k) {
-                        const int lv = decode4<4>((wd >> (4 * k)) & 0x0f0f0f0fu, lut);
-#pragma unroll
-                        for (int t = 0; t < T; ++t) {
-                            const int a =
-                                *reinterpret_cast<const int*>(xq_s + (size_t)t * p.padded + 32 * c + 8 * d + 4 * k);
-                            part[t] = dot4(lv, a, part[t]);
-                        }
+                        const int lv = decode4<4>(wd >> (4 * k), lut);
+                        part = dot4(lv, *reinterpret_cast<const int*>(xq_s + 32 * c + 8 * d + 4 * k), part);
                     }
                 }
             }
-            const bool store = (lane % CPG) == 0 && idx < R * CPR && rw + rl < p.rows;
-#pragma unroll
-            for (int t = 0; t < T; ++t) {
-                const int s = set_sum<CPG>(part[t]);
-                if (store) acc_s[((size_t)t * R + rl) * G + c / CPG] = s;
-            }
+            const int s = set_sum<CPG>(part);
+            if ((lane % CPG) == 0 && idx < R * CPR && rw + rl < p.rows) acc_s[rl * G + c / CPG] = s;
             // one chunk's code reads at a time: hoisting them all would hold
             // 16 registers a chunk and cut the waves a CU keeps in flight
             __builtin_amdgcn_sched_barrier(0);
@@ -363,13 +345,12 @@ __device__ __forceinline__ void cb_product_body(const CodebookParams& p, const f
         __builtin_amdgcn_wave_barrier();  // acc_s is this wave's own
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 
-        // 4. sequential epilogue per (token, row)
-        for (int e = lane; e < T * R; e += 64) {
-            const int t = e / R, r = e - t * R;
-            if (rw + r >= p.rows || t0 + t >= count) continue;
-            const int* a = acc_s + ((size_t)t * R + r) * G;
+        // 4. sequential epilogue per row
+        for (int r = lane; r < R; r += 64) {
+            if (rw + r >= p.rows) continue;
+            const int* a = acc_s + r * G;
             const uint16_t* nm = nm_s + nhalf0 + (wv * R + r) * G;
-            const float* xs = sx_s + t * G;
+            const float* xs = sx_s;
             float total = 0.0f;
             for (int g = 0; g < G; ++g) {
                 const float norm = half_bits_to_float(nm[g]);
@@ -378,9 +359,10 @@ __device__ __forceinline__ void cb_product_body(const CodebookParams& p, const f
                 else
                     total = total + ((((float)a[g] * norm) * p.lscale) * xs[g]);  // neon.rs:158,180
             }
-            y[(size_t)(t0 + t) * p.rows + rw + r] = total;
+            const size_t o = (size_t)blockIdx.y * p.rows + rw + r;
+            y[o] = total;
             if (acc_out != nullptr)
-                for (int g = 0; g < G; ++g) acc_out[((size_t)(t0 + t) * p.rows + rw + r) * G + g] = a[g];
+                for (int g = 0; g < G; ++g) acc_out[o * G + g] = a[g];
         }
         __syncthreads();  // the norms window and acc_s are read before the next row group replaces them
     };
@@ -394,10 +376,10 @@ __device__ __forceinline__ void cb_product_body(const CodebookParams& p, const f
     }
 }
 
-template <int BITS, int GROUP, int FORM, int NL, int T>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NL == 8 && T == 1 ? 3 : 1)))
-void cb_product_kernel(CodebookParams p, const float* x, int count, float* y, int32_t* acc_out) {
-    cb_product_body<BITS, GROUP, FORM, NL, T>(p, x, count, y, acc_out);
+template <int BITS, int GROUP, int FORM, int NL>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NL == 8 ? 3 : 1)))
+void cb_product_kernel(CodebookParams p, const float* x, float* y, int32_t* acc_out) {
+    cb_product_body<BITS, GROUP, FORM, NL>(p, x, y, acc_out);
 }
 
 // Up to four products of one shape in one launch (blockIdx.z picks the job):
@@ -406,27 +388,254 @@ template <int BITS, int GROUP, int FORM, int NL>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NL == 8 ? 3 : 1)))
 void cb_product_jobs_kernel(CodebookJobs jobs) {
     const CodebookJob& j = jobs.job[blockIdx.z];
-    cb_product_body<BITS, GROUP, FORM, NL, 1>(j.p, j.x, 1, j.y, nullptr);
+    cb_product_body<BITS, GROUP, FORM, NL>(j.p, j.x, j.y, nullptr);
+}
+
+// The products of a batch on the matrix cores: up to 16 SM tokens (blockIdx.y)
+// by a range of 16-row sub-tiles (blockIdx.x), eight waves a block.
+//
+// One v_mfma_i32_16x16x64_i8 covers 64 columns of a 16-token x 16-row sub-tile,
+// so a group's exact int32 sums take GROUP / 64 of them, chained through the
+// accumulator, and land in the lane's registers, where the sequential group
+// epilogue runs: no sum goes through LDS or across lanes. Lane (r, q) (r = lane
+// % 16, q = lane / 16) holds row r's runs of 16 columns q * GROUP / 64 .. of a
+// group, decoded in plane order, the order in which the token codes lie in LDS,
+// so the two operands meet element by element.
+//   1. The wave's first weights and norms are requested, then the block's token
+//      rows are quantised per group into LDS (the codes of all columns, row
+//      pitch padded + 16 bytes: the 16 rows of a fragment read fall in distinct
+//      bank groups).
+//   2. Each wave takes every eighth sub-tile of the block's range, 128 bytes of
+//      every row at a time: 16-byte pieces of consecutive row bytes, two such
+//      batches in flight in registers, through the wave's own LDS slot (reading
+//      a lane's few bytes of 16 rows straight from memory measured slower: 16
+//      cache lines a request). A sub-tile's norms are 32 G consecutive bytes,
+//      requested one sub-tile ahead.
+// A block's quantisation (15 vector operations a value, repeated by every block
+// of a token tile) and the latency of its first loads bound a prompt chunk, the
+// decode and the epilogue (23 vector operations a product at 4 bits) the largest.
+// Measured per call, against tiles of eight tokens on v_dot4: 256 tokens x 2048
+// rows x 768 columns of 2 bits 7.2 us (was 53), 512 x 8192 x 768 18 us (was
+// 330), 4-bit 512 x 8192 x 4096 110 us, 314 TOPS (was 2110).
+constexpr int kTileWaves = 8;
+constexpr int kTileBatch = 128;                            // bytes of a row per batch
+constexpr int kTileSlot = 16 * (kTileBatch + 16);          // a wave's batch in LDS: rows 16 bytes apart in banks
+constexpr int kTileNormLoads = 4;                          // 16-byte pieces of norms a lane: up to 128 groups
+
+template <int BITS, int GROUP, int FORM, int SM, bool DUMP>
+__global__ __launch_bounds__(64 * kTileWaves) void cb_tile_kernel(CodebookParams p, const float* x, int count, float* y,
+                                                                  int32_t* acc_out, int subs, int tile) {
+    constexpr int IB = BITS == 5 ? 2 : BITS;
+    constexpr int BM = 16 * SM, NT = 64 * kTileWaves;
+    constexpr int RPG = GROUP / 16, QR = GROUP / 64;  // runs of a group, a lane's runs of it
+    constexpr int GB = GROUP * IB / 8;                // a row's bytes of a group
+    constexpr int NG = kTileBatch / GB;               // groups of a batch
+    static_assert(NG >= 1, "whole groups a batch");
+    extern __shared__ __align__(16) unsigned char lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int G = p.padded / GROUP, runs = p.padded / 16, pitch = p.padded + 16;
+    const int t0 = blockIdx.y * tile, live = min(tile, count - t0);
+    int8_t* xq_s = reinterpret_cast<int8_t*>(lds);                                  // [BM][pitch]
+    float* sx_s = reinterpret_cast<float*>(lds + (size_t)BM * pitch);               // [G][BM]
+    unsigned char* w_s = lds + (size_t)BM * (pitch + 4 * G) + wave * kTileSlot;      // this wave's weights
+    unsigned char* n_s = lds + (size_t)BM * (pitch + 4 * G) + kTileWaves * kTileSlot + wave * 32 * G;  // and norms
+
+    const int r16 = lane & 15, q = lane >> 4;
+    const int batches = (p.row_bytes + 2 * kTileBatch - 1) / (2 * kTileBatch) * 2;  // in pairs
+    const int sub0 = blockIdx.x * subs + wave, sub_end = min((int)(blockIdx.x + 1) * subs, (p.rows + 15) / 16);
+    const int mine = sub0 < sub_end ? (sub_end - sub0 + kTileWaves - 1) / kTileWaves : 0;
+    struct Batch {
+        v4i piece[2];
+    };
+    // pieces 8 lanes a row, 8 rows an instruction; rows and bytes past the end repeat the last
+    auto issue = [&](int s, int b, Batch& o) {
+        if (b >= batches) b -= batches, ++s;
+        const int base = (sub0 + kTileWaves * min(s, mine - 1)) * 16;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int row = min(base + 8 * j + (lane >> 3), p.rows - 1);
+            const int byte = min(kTileBatch * b + 16 * (lane & 7), p.row_bytes - 16);
+            o.piece[j] = *reinterpret_cast<const v4i*>(p.packed + (size_t)row * p.row_bytes + byte);
+        }
+    };
+    v4i nv[kTileNormLoads];
+    auto issue_norms = [&](int s) {
+        const int base = (sub0 + kTileWaves * min(s, mine - 1)) * 16;
+        const unsigned char* src = reinterpret_cast<const unsigned char*>(p.norms) + (size_t)base * G * 2;
+#pragma unroll
+        for (int j = 0; j < kTileNormLoads; ++j)
+            nv[j] = *reinterpret_cast<const v4i*>(src + 16 * min(64 * j + lane, 2 * G - 1));
+    };
+    Batch wa, wb;
+    if (mine > 0) {
+        issue(0, 0, wa);
+        issue(0, 1, wb);
+        issue_norms(0);
+    }
+
+    // 1. the tile's codes and scales (tokens past the batch keep whatever LDS
+    // holds: their sums are never stored)
+    const int xruns = live * runs;
+    auto load_run = [&](int f, float (&v)[16]) {
+        const float4* src = reinterpret_cast<const float4*>(x + (size_t)t0 * p.padded + 16 * (size_t)min(f, xruns - 1));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float4 f4 = src[i];
+            v[4 * i] = f4.x;
+            v[4 * i + 1] = f4.y;
+            v[4 * i + 2] = f4.z;
+            v[4 * i + 3] = f4.w;
+        }
+    };
+    auto quantise_run = [&](int f, float (&v)[16]) {
+        float peak = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) peak = fmaxf(peak, fabsf(v[i]));
+        peak = set_max<RPG>(peak);
+        const float sx = int8_scale_from_peak(peak);
+        float quot[16];
+        quotients<16>(v, sx, quot);
+        int c[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) c[i] = code_of_quotient(quot[i]);
+        if (f < xruns) {
+            const int t = f / runs, u = f - t * runs;
+            *reinterpret_cast<int4*>(xq_s + (size_t)t * pitch + 16 * u) = plane_pack<IB>(c);
+            if (u % RPG == 0) sx_s[(u / RPG) * BM + t] = sx;
+        }
+    };
+    float va[16], vb[16];
+    load_run(tid, va);
+    load_run(tid + NT, vb);
+    for (int f = tid; f - tid < xruns; f += 2 * NT) {  // the next two runs arrive under this one's quantisation
+        float na[16], nb[16];
+        load_run(f + 2 * NT, na);
+        load_run(f + 3 * NT, nb);
+        quantise_run(f, va);
+        if (f - tid + NT < xruns) quantise_run(f + NT, vb);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) va[i] = na[i], vb[i] = nb[i];
+    }
+    __syncthreads();
+
+    // 2. the group chains
+    const uint32_t lut[4] = {p.lut[0], p.lut[1], p.lut[2], p.lut[3]};
+    const int8_t* a_s = xq_s + (size_t)r16 * pitch + q * (16 * QR);
+    const unsigned char* b_s = w_s + r16 * (kTileBatch + 16) + q * (GB / 4);
+    const uint16_t* norm_s = reinterpret_cast<const uint16_t*>(n_s) + r16 * G;
+    const float* xs_s = sx_s + 4 * q;
+    float total[SM][4];
+    // U groups from group j of batch b: every product before the first epilogue
+    auto groups = [&](auto unit, int row, int b, int j) {
+        constexpr int U = decltype(unit)::value;
+        const int g0 = b * NG + j;
+        v4i acc[U][SM];
+#pragma unroll
+        for (int k = 0; k < U; ++k) {
+#pragma unroll
+            for (int m = 0; m < SM; ++m) acc[k][m] = v4i{0, 0, 0, 0};
+            uint32_t wd[QR * IB / 2];
+            __builtin_memcpy(wd, __builtin_assume_aligned(b_s + (j + k) * GB, 2 * QR * IB > 16 ? 16 : 2 * QR * IB), 2 * QR * IB);
+#pragma unroll
+            for (int u = 0; u < QR; ++u) {
+                v4i bf;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if constexpr (IB == 2)
+                        bf[e] = decode4<2>((wd[u] >> (2 * e)) & 0x03030303u, lut);
+                    else
+                        bf[e] = decode4<4>(wd[2 * u + e / 2] >> (4 * (e & 1)), lut);
+                }
+#pragma unroll
+                for (int m = 0; m < SM; ++m) {
+                    const v4i af = *reinterpret_cast<const v4i*>(a_s + (size_t)(16 * m) * pitch + (g0 + k) * GROUP + 16 * u);
+                    acc[k][m] = __builtin_amdgcn_mfma_i32_16x16x64_i8(af, bf, acc[k][m], 0, 0, 0);
+                }
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < U; ++k) {
+            const float norm = half_bits_to_float(norm_s[g0 + k]);
+            const float nl = norm * p.lscale;
+#pragma unroll
+            for (int m = 0; m < SM; ++m) {
+                const float4 xs4 = *reinterpret_cast<const float4*>(xs_s + (g0 + k) * BM + 16 * m);
+                const float xs[4] = {xs4.x, xs4.y, xs4.z, xs4.w};
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    if constexpr (FORM == kPanel)
+                        total[m][i] = fmaf((float)acc[k][m][i], nl * xs[i], total[m][i]);  // panel.rs:184-188
+                    else
+                        total[m][i] = total[m][i] + ((((float)acc[k][m][i] * norm) * p.lscale) * xs[i]);  // neon.rs:158,180
+                }
+                if (DUMP && row < p.rows) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const int t = 16 * m + 4 * q + i;
+                        if (t < live) acc_out[((size_t)(t0 + t) * p.rows + row) * G + g0 + k] = acc[k][m][i];
+                    }
+                }
+            }
+        }
+    };
+    auto compute = [&](int s, int row, int b, Batch& o) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+            *reinterpret_cast<v4i*>(w_s + (8 * j + (lane >> 3)) * (kTileBatch + 16) + 16 * (lane & 7)) = o.piece[j];
+        issue(s, b + 2, o);
+        wave_lds_sync();
+        const int have = min(NG, G - b * NG);  // uniform
+#pragma unroll
+        for (int j = 0; j < NG; j += 2) {
+            if (j + 1 < have) groups(std::integral_constant<int, NG >= 2 ? 2 : 1>(), row, b, j);
+            else if (j < have) groups(std::integral_constant<int, 1>(), row, b, j);
+        }
+        wave_lds_sync();
+    };
+    for (int s = 0; s < mine; ++s) {
+        const int row = (sub0 + kTileWaves * s) * 16 + r16;
+#pragma unroll
+        for (int j = 0; j < kTileNormLoads; ++j)
+            if (64 * j + lane < 2 * G) reinterpret_cast<v4i*>(n_s)[64 * j + lane] = nv[j];
+        issue_norms(s + 1);
+#pragma unroll
+        for (int m = 0; m < SM; ++m)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) total[m][i] = 0.0f;
+        for (int b = 0; b < batches; b += 2) {
+            compute(s, row, b, wa);
+            compute(s, row, b + 1, wb);
+        }
+        if (row < p.rows) {
+#pragma unroll
+            for (int m = 0; m < SM; ++m)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int t = 16 * m + 4 * q + i;
+                    if (t < live) y[(size_t)(t0 + t) * p.rows + row] = total[m][i];
+                }
+        }
+    }
 }
 
 namespace {
 
-// LDS of a product block: norms window, [T][padded] codes, [4][T][R][G] sums, [T][G] scales
-inline size_t product_lds(const CodebookParams& p, int T, int R) {
+// LDS of a product block: norms window, [padded] codes, [4][R][G] sums, [G] scales
+inline size_t product_lds(const CodebookParams& p, int R) {
     const size_t G = (size_t)(p.padded / p.group);
-    return kNormWindow + (size_t)T * p.padded + 4 * (4 * (size_t)T * R * G + (size_t)T * G);
+    return kNormWindow + p.padded + 4 * (4 * R * G + G);
 }
 inline int product_loads(const CodebookParams& p) { return p.cpr < 64 ? 8 : 16; }
 inline int product_rows(const CodebookParams& p) { return min(64, 64 * product_loads(p) / p.cpr); }
 constexpr size_t kProductMaxLds = 64 * 1024;
 
-template <int BITS, int GROUP, int FORM, int T>
-hipError_t launch_product_t(const CodebookParams& p, const float* x, int count, float* y, int32_t* acc,
+template <int BITS, int GROUP, int FORM>
+hipError_t launch_product_rows(const CodebookParams& p, const float* x, int count, float* y, int32_t* acc,
                             hipStream_t stream) {
     const int nl = product_loads(p);
     CodebookParams q = p;
     q.rows_per_block = product_rows(p);
-    const size_t lds = product_lds(p, T, q.rows_per_block);
+    const size_t lds = product_lds(p, q.rows_per_block);
     if (lds > kProductMaxLds) return hipErrorInvalidValue;
     // consecutive row groups per block (at least 4, or padded / 1024 for a wide
     // input, whose prologue then serves them all), while the grid keeps at
@@ -434,22 +643,59 @@ hipError_t launch_product_t(const CodebookParams& p, const float* x, int count, 
     // group's decode
     const int groups = (p.rows + 4 * q.rows_per_block - 1) / (4 * q.rows_per_block);
     q.iters = max(1, min(max(4, p.padded / 1024), groups / 512));
-    const dim3 grid((groups + q.iters - 1) / q.iters, (count + T - 1) / T);
+    const dim3 grid((groups + q.iters - 1) / q.iters, count);
     if (nl == 8)
-        rn_launch(cb_product_kernel<BITS, GROUP, FORM, 8, T>, grid, dim3(256), lds, stream, q, x, count, y, acc);
+        rn_launch(cb_product_kernel<BITS, GROUP, FORM, 8>, grid, dim3(256), lds, stream, q, x, y, acc);
     else
-        rn_launch(cb_product_kernel<BITS, GROUP, FORM, 16, T>, grid, dim3(256), lds, stream, q, x, count, y, acc);
+        rn_launch(cb_product_kernel<BITS, GROUP, FORM, 16>, grid, dim3(256), lds, stream, q, x, y, acc);
+    return hipGetLastError();
+}
+
+// LDS of a token tile of the matrix-core kernel: [bm][padded + 16] codes, [G][bm]
+// scales, then each wave's weights and norms
+inline size_t tile_lds(const CodebookParams& p, int bm) {
+    const size_t G = (size_t)(p.padded / p.group);
+    return (size_t)bm * (p.padded + 16 + 4 * G) + kTileWaves * (kTileSlot + 32 * G);
+}
+constexpr size_t kTileMaxLds = 144 * 1024;
+
+template <int BITS, int GROUP, int FORM, int SM, bool DUMP = false>
+hipError_t launch_tile(const CodebookParams& p, const float* x, int count, float* y, int32_t* acc, hipStream_t stream) {
+    const int subs = (p.rows + 15) / 16;
+    // fewer tokens a tile while that leaves most of the chip idle: a block
+    // quantises only its own (the product's unused columns cost nothing then)
+    int tile = 16 * SM;
+    auto tiles = [&]() { return (count + tile - 1) / tile; };
+    if (SM == 1)
+        while (tile > 1 && tiles() * ((subs + 7) / 8) <= 64) tile /= 2;
+    // row ranges of whole rounds of the eight waves, one block a CU where the rows allow it
+    const int blocks = max(1, min((subs + 7) / 8, 256 / tiles()));
+    const int per = ((subs + blocks - 1) / blocks + 7) / 8 * 8;
+    rn_launch((cb_tile_kernel<BITS, GROUP, FORM, SM, DUMP>), dim3((subs + per - 1) / per, tiles()), dim3(512),
+              tile_lds(p, 16 * SM), stream, p, x, count, y, acc, per, tile);
     return hipGetLastError();
 }
 
 template <int BITS, int GROUP, int FORM>
 hipError_t launch_product_g(const CodebookParams& p, const float* x, int count, float* y, int32_t* acc,
                             hipStream_t stream) {
-    // token tiles of 8 share each block's weight loads; one token a block when
-    // 8 tokens' codes would not fit the LDS budget
-    const bool tile = count > 1 && product_lds(p, 8, product_rows(p)) <= kProductMaxLds;
-    return tile ? launch_product_t<BITS, GROUP, FORM, 8>(p, x, count, y, acc, stream)
-                : launch_product_t<BITS, GROUP, FORM, 1>(p, x, count, y, acc, stream);
+    // One token a block while the whole batch is small: the blocks then outnumber
+    // the tile kernel's and each quantises one row (5.4 against 5.8 us at 16
+    // tokens x 2000 rows x 1024 columns of 2 bits, 6.4 against 5.1 us at 64 x
+    // 2000 x 384; 9.7 against 8.6 at 16 x 2000 x 2560). Rows too wide for a tile's
+    // LDS stay there too.
+    const long long weights = (long long)count * p.rows * p.padded;
+    const bool fits = p.padded / p.group <= 32 * kTileNormLoads && tile_lds(p, 16) <= kTileMaxLds;
+    if (count == 1 || !fits || (weights <= (1ll << 25) && count <= 65535))
+        return launch_product_rows<BITS, GROUP, FORM>(p, x, count, y, acc, stream);
+    if (acc != nullptr) return launch_tile<BITS, GROUP, FORM, 1, true>(p, x, count, y, acc, stream);
+    // two 16-token sub-tiles a wave halve the decode per product and double the
+    // block's quantisation: they pay once a block has some hundred rows (4-bit
+    // indices cost three times the 2-bit decode)
+    const bool wide = count > 16 && (long long)p.rows * count > (p.bits == 4 ? 1ll << 20 : 3ll << 20) &&
+                      tile_lds(p, 32) <= kTileMaxLds;
+    return wide ? launch_tile<BITS, GROUP, FORM, 2>(p, x, count, y, acc, stream)
+                : launch_tile<BITS, GROUP, FORM, 1>(p, x, count, y, acc, stream);
 }
 
 template <int BITS, int FORM>
@@ -583,7 +829,7 @@ template <int BITS, int GROUP, int FORM>
 hipError_t launch_jobs_t(CodebookJobs jobs, int n, hipStream_t stream) {
     const CodebookParams& p = jobs.job[0].p;
     const int nl = product_loads(p), R = product_rows(p);
-    const size_t lds = product_lds(p, 1, R);
+    const size_t lds = product_lds(p, R);
     if (lds > kProductMaxLds) return hipErrorInvalidValue;
     const int groups = (p.rows + 4 * R - 1) / (4 * R);
     const int iters = max(1, min(max(4, p.padded / 1024), groups / 512));

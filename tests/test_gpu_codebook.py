@@ -61,6 +61,30 @@ def test_batch_product(bits, group, rows, columns, count):
     assert np.array_equal(_bits(y), _bits(yo))
 
 
+# batches past the one-token-a-block size: tokens, rows and columns around the
+# 16-token tile, its narrower and wider forms, the eight waves' rounds of 16-row
+# sub-tiles, the 128-byte batches of a row and the pieces of the norms
+@pytest.mark.parametrize("bits,group,rows,columns,count", [
+    (2, 128, 2001, 1000, 17),    # one token past a tile, a ragged last sub-tile
+    (2, 128, 2048, 1100, 16),    # two tokens a tile
+    (4, 64, 517, 4096, 31),      # 64 groups a row: two pieces of norms a lane
+    (5, 256, 300, 7000, 33),     # a batch of two 256-column groups, padded width
+    (4, 256, 1030, 600, 128),    # one group fills a batch
+    (2, 64, 8005, 64, 401),      # 32-token tiles, one group a row
+    (4, 128, 9001, 130, 130),    # 32-token tiles of 4-bit indices
+])
+def test_batch_product_on_the_matrix_cores(bits, group, rows, columns, count):
+    g, o = _pair(bits, group, rows, columns, seed=count)
+    x = rn.synth_normal(9, "cbt", 1.0, (count, columns))
+    x[count - 1] *= 1e3
+    x[count // 2] = 0.0
+    rotated = g.prepare_host(x)
+    yo, acco = o.multiply_rotated(rotated, with_acc=True)
+    assert np.array_equal(_bits(g.multiply_batch_host(rotated)), _bits(yo))
+    y, acc = g.multiply_batch_host(rotated, with_acc=True)
+    assert np.array_equal(acc, acco) and np.array_equal(_bits(y), _bits(yo))
+
+
 def test_zero_and_sparse_inputs():
     g, o = _pair(2, 128, 96, 512, seed=1)
     x = np.zeros((2, 512), np.float32)
