@@ -750,6 +750,250 @@ __global__ __launch_bounds__(256) void n3_attend_kernel(N3AttendParams p) {
     }
 }
 
+// n3_attend_kernel for a run of `count` tokens on the matrix cores: query head
+// blockIdx.x of the `tile` tokens (a power of two, at most 16) from blockIdx.y *
+// tile, 512 threads, over every position any of them sees. Both contractions are
+// exact integers, so their order is free: the scores are one
+// v_mfma_i32_16x16x64_i8 per 16 tokens x 16 positions, the 12-bit weights enter as
+// two int8 digits (w = 128 hi + lo) against the value codes, 64 positions an
+// instruction, transposed to a lane's dimension with byte permutes. What stays
+// sequential is each token's four exponent sums: one wave runs the tile's 4 x 16
+// chains, a lane each, while the others take the value steps (handed out by a
+// counter in LDS, so that wave joins when it is done).
+//   1. scores and coefficients into e_s [tile][pitch] (-inf where a token does not
+//      see the position), the peaks; the value scales into vs_s;
+//   2. exponents in place (0 outside a token's range), the peaks of e * value scale;
+//   3. the exponent totals; the weights and the value sums;
+//   4. scaling, 1 / total and the output gate per (token, dimension).
+// Bound by its vector work, about 45 operations a (token, position) pair.
+// Measured: 256 tokens x 12 heads in a 2000-token feed, 15.3 us a launch (a block a
+// (head, token) on v_dot4 took 73, its value sums and the four lone chains in turn).
+constexpr int kN3TileThreads = 512;
+
+// Bytes of LDS of a tile over rows of `pitch` floats.
+inline size_t n3_attend_tile_lds(int tile, int pitch) {
+    return sizeof(float) * (size_t)(tile + 1) * pitch + sizeof(int) * 16 * kN3Head;
+}
+
+__global__ __launch_bounds__(kN3TileThreads) void n3_attend_tile_kernel(N3AttendParams p, int count, int tile, int pitch) {
+    constexpr int NW = kN3TileThreads / 64;
+    extern __shared__ __align__(16) float tile_lds[];
+    __shared__ float peak_s[NW][16], cpeak_s[NW][16], total_s[16];
+    __shared__ int next_s;
+    float* const e_s = tile_lds;                       // [tile][pitch]
+    float* const vs_s = tile_lds + (size_t)tile * pitch;  // [pitch]
+    int* const sum_s = reinterpret_cast<int*>(vs_s + pitch);  // [16][64]
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r16 = lane & 15, q = lane >> 4;
+    const int h = blockIdx.x, H = gridDim.x, kvh = h / p.group, t0 = blockIdx.y * tile, live = min(tile, count - t0);
+    // token t sees positions first_of(t) .. p.position + t0 + t
+    auto first_of = [&](int t) {
+        const int total = p.position + t0 + t + 1;
+        return p.window > 0 && total > p.window ? total - p.window : 0;
+    };
+    const int lo = first_of(0), hi = p.position + t0 + live, span = (hi - lo + 63) & ~63;
+    const int8_t* const keys = p.keys + (size_t)kvh * p.cap * kN3Head;
+    const int8_t* const values = p.values + (size_t)kvh * p.cap * kN3Head;
+    const float* const ks = p.key_scales + (size_t)kvh * p.cap;
+    const float* const vs = p.value_scales + (size_t)kvh * p.cap;
+    auto row16_max = [](float v) {  // over the 16 lanes of a q
+        v = fmaxf(v, __int_as_float(dpp_move<0xb1>(__float_as_int(v))));
+        v = fmaxf(v, __int_as_float(dpp_move<0x4e>(__float_as_int(v))));
+        v = fmaxf(v, __int_as_float(dpp_move<0x141>(__float_as_int(v))));
+        return fmaxf(v, __int_as_float(dpp_move<0x140>(__float_as_int(v))));
+    };
+
+    // 1. this lane's tokens are 4 q + i, its positions n + r16
+    const v4i aq = *reinterpret_cast<const v4i*>(p.qcodes + ((size_t)(t0 + min(r16, live - 1)) * H + h) * kN3Head + 16 * q);
+    float qsc[4];
+    int first[4], last[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int t = 4 * q + i;
+        qsc[i] = p.qscales[(size_t)(t0 + min(t, live - 1)) * H + h] * p.inverse_root;
+        first[i] = first_of(t);
+        last[i] = t < live ? p.position + t0 + t : -1;
+    }
+    float peak[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+    constexpr int U = 4;  // sub-tiles of keys in flight
+    for (int n0 = 16 * wave; n0 < span; n0 += 16 * NW * U) {
+        v4i kf[U];
+        float sc[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int pos = min(lo + n0 + 16 * NW * u + r16, hi - 1);
+            kf[u] = *reinterpret_cast<const v4i*>(keys + (size_t)pos * kN3Head + 16 * q);
+            sc[u] = ks[pos];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int n = n0 + 16 * NW * u;
+            if (n < span) {
+                const v4i acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(aq, kf[u], v4i{0, 0, 0, 0}, 0, 0, 0);
+                const int pos = lo + n + r16;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float c = ((float)acc[i] * sc[u]) * qsc[i];
+                    const bool seen = pos >= first[i] && pos <= last[i];
+                    if (seen) peak[i] = fmaxf(peak[i], c);
+                    if (4 * q + i < tile) e_s[(size_t)(4 * q + i) * pitch + n + r16] = seen ? c : -INFINITY;
+                }
+            }
+        }
+    }
+    for (int n = tid; n < span; n += kN3TileThreads) vs_s[n] = vs[min(lo + n, hi - 1)];
+    for (int n = tid; n < 16 * kN3Head; n += kN3TileThreads) sum_s[n] = 0;
+    if (tid == 0) next_s = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        peak[i] = row16_max(peak[i]);
+        if (r16 == 0) peak_s[wave][4 * q + i] = peak[i];
+    }
+    __syncthreads();
+
+    // 2.
+    float cpeak[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int w = 0; w < NW; ++w) peak[i] = fmaxf(peak[i], peak_s[w][4 * q + i]);
+    for (int n = 16 * wave; n < span; n += 16 * NW) {
+        const int pos = lo + n + r16;
+        const float v = vs_s[n + r16];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (4 * q + i < tile) {
+                float* const slot = e_s + (size_t)(4 * q + i) * pitch + n + r16;
+                const bool seen = pos >= first[i] && pos <= last[i];
+                const float e = seen ? fast_exp(*slot - peak[i]) : 0.0f;
+                *slot = e;
+                if (seen) cpeak[i] = fmaxf(cpeak[i], fabsf(e * v));
+            }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        cpeak[i] = row16_max(cpeak[i]);
+        if (r16 == 0) cpeak_s[wave][4 * q + i] = cpeak[i];
+    }
+    __syncthreads();
+    auto coefficient_peak = [&](int t) {
+        float c = cpeak_s[0][t];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) c = fmaxf(c, cpeak_s[w][t]);
+        return c;
+    };
+    // a normal scale keeps every weight within 0..2047; a row whose scale is
+    // not (values of almost no magnitude) takes its sums one by one in step 4
+    constexpr float kPlain = 0x1p-114f;
+
+    // 3. the totals: lane 4 t + j runs lane sum j of token t (neon.rs:278-311)
+    if (wave == 0) {
+        const int t = lane >> 2, j = lane & 3;
+        if (t < live) {
+            const int begin = first_of(t), have = p.position + t0 + t + 1 - begin, vector_count = have - have % 4;
+            const float* const e = e_s + (size_t)t * pitch + (begin - lo);
+            float s = 0.0f;
+            int k = j;
+            for (; k + 64 <= vector_count; k += 64) {
+                float v[16];
+#pragma unroll
+                for (int m = 0; m < 16; ++m) v[m] = e[k + 4 * m];
+#pragma unroll
+                for (int m = 0; m < 16; ++m) s = s + v[m];
+            }
+            for (; k < vector_count; k += 4) s = s + e[k];
+            const int b = __float_as_int(s);
+            float total = (__int_as_float(dpp_move<0x00>(b)) + __int_as_float(dpp_move<0x55>(b))) +
+                          (__int_as_float(dpp_move<0xaa>(b)) + __int_as_float(dpp_move<0xff>(b)));
+            for (int m = vector_count; m < have; ++m) total = total + e[m];
+            if (j == 0) total_s[t] = total;
+        }
+    }
+    // the weights (token r16, positions n + 16 q ..) and the value sums
+    // (tokens 4 q + i, dimensions 4 r16 + k)
+    const int row = r16 & (tile - 1);
+    const float cp = coefficient_peak(row), scale = cp >= kPlain ? cp / 2047.0f : 1.0f;
+    v4i high[4], low[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) high[k] = low[k] = v4i{0, 0, 0, 0};
+    for (;;) {
+        int step = 0;
+        if (lane == 0) step = atomicAdd(&next_s, 1);
+        const int n = 64 * __builtin_amdgcn_readfirstlane(step);
+        if (n >= span) break;
+        uint32_t vd[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const int pos = min(lo + n + 16 * q + j, hi - 1);
+            vd[j] = *reinterpret_cast<const uint32_t*>(values + (size_t)pos * kN3Head + 4 * r16);
+        }
+        float v[16], y[16];
+        const float4* const e4 = reinterpret_cast<const float4*>(e_s + (size_t)row * pitch + n + 16 * q);
+        const float4* const s4 = reinterpret_cast<const float4*>(vs_s + n + 16 * q);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float4 e = e4[j], s = s4[j];
+            v[4 * j] = e.x * s.x;
+            v[4 * j + 1] = e.y * s.y;
+            v[4 * j + 2] = e.z * s.z;
+            v[4 * j + 3] = e.w * s.w;
+        }
+        quotients<16>(v, scale, y);
+        v4i wh, wl;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            uint32_t a = 0, b = 0;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const uint32_t w = (uint32_t)(int)__builtin_roundf(y[4 * j + k]);
+                a |= (w >> 7) << (8 * k);
+                b |= (w & 127u) << (8 * k);
+            }
+            wh[j] = (int)a;
+            wl[j] = (int)b;
+        }
+        v4i vf[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {  // 4 positions x 4 dimensions of bytes, transposed
+            const uint32_t x0 = vd[4 * j], x1 = vd[4 * j + 1], x2 = vd[4 * j + 2], x3 = vd[4 * j + 3];
+            const uint32_t a0 = __builtin_amdgcn_perm(x1, x0, 0x05010400u), a1 = __builtin_amdgcn_perm(x3, x2, 0x05010400u);
+            const uint32_t b0 = __builtin_amdgcn_perm(x1, x0, 0x07030602u), b1 = __builtin_amdgcn_perm(x3, x2, 0x07030602u);
+            vf[0][j] = (int)__builtin_amdgcn_perm(a1, a0, 0x05040100u);
+            vf[1][j] = (int)__builtin_amdgcn_perm(a1, a0, 0x07060302u);
+            vf[2][j] = (int)__builtin_amdgcn_perm(b1, b0, 0x05040100u);
+            vf[3][j] = (int)__builtin_amdgcn_perm(b1, b0, 0x07060302u);
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            high[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wh, vf[k], high[k], 0, 0, 0);
+            low[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wl, vf[k], low[k], 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) atomicAdd(&sum_s[(4 * q + i) * kN3Head + 4 * r16 + k], 128 * high[k][i] + low[k][i]);
+    __syncthreads();
+
+    // 4.
+    for (int o = tid; o < live * kN3Head; o += kN3TileThreads) {
+        const int t = o / kN3Head, dim = o % kN3Head;
+        const float c = coefficient_peak(t), sc = c / 2047.0f;
+        int sum = sum_s[o];
+        if (c > 0.0f && c < kPlain) {
+            sum = 0;
+            for (int pos = first_of(t); pos <= p.position + t0 + t; ++pos) {
+                const int w = (int)__builtin_roundf((e_s[(size_t)t * pitch + pos - lo] * vs_s[pos - lo]) / sc);
+                sum += w * (int)values[(size_t)pos * kN3Head + dim];
+            }
+        }
+        float r = c > 0.0f ? (float)sum * sc : 0.0f;
+        r = r * reciprocal(total_s[t]);
+        r = r * libm_sigmoid(p.gate[(size_t)(t0 + t) * p.gate_stride + (size_t)h * kN3Head + dim]);
+        p.out[((size_t)(t0 + t) * H + h) * kN3Head + dim] = r;
+    }
+}
+
 // ops.rs:120-125 over n <= 4096 values (one block a vector: block b reads in +
 // b * n), then, for group > 0, prepare for a matrix of that group and padded
 // width (matrix.rs:123-128) into out + b * padded (else out + b * n)
@@ -3763,7 +4007,16 @@ int enqueue_run(rn_n3_session* s, const uint32_t* tokens, int count) {
         }
         N3AttendParams ap{r.qcodes, r.qscales, c.keys, c.key_scales, c.values, c.value_scales, r.prod + qkv,
                           s->capacity, P0, layer_window(g, layer), H / KV, 1.0f / sqrtf(64.0f), r.attended, rows};
-        rn_launch(n3_attend_kernel, dim3(H, T), dim3(256), 0, st, ap);
+        // 16 tokens a block, fewer where their rows would not fit the LDS; rows
+        // 4 floats past a multiple of 64, so that neighbours start on other banks
+        int tile = 16, pitch = 0;
+        for (;; tile /= 2) {
+            const int span = std::min(P0 + T, ap.window > 0 ? ap.window + tile - 1 : P0 + T);
+            pitch = (span + 63) / 64 * 64 + 4;
+            if (tile == 1 || n3_attend_tile_lds(tile, pitch) <= 144 * 1024) break;
+        }
+        rn_launch(n3_attend_tile_kernel, dim3(H, (T + tile - 1) / tile), dim3(kN3TileThreads), n3_attend_tile_lds(tile, pitch),
+                  st, ap, T, tile, pitch);
         N3_HIP(hipGetLastError());
         rn_launch(n3_fake_quantise_kernel, dim3(T), dim3(kN3Block), 0, st, (const float*)r.attended, qw,
                   y.out->cb.padded, y.out->group, y.out->cb.wht_scale, r.rotated);

@@ -263,3 +263,46 @@ def test_float_path_projections_feed_as_the_reference_prefills(path):
         os_.push(t)
     assert gs.decode_greedy(9, 4).tolist() == os_.greedy(9, 4).tolist()
     _compare_all(gs, os_, gm, "3-bit after pushes and greedy tokens")
+
+
+def test_long_feed_equals_pushes(archive):
+    """A feed whose attention tiles hold 16, 8, 4 and then 2 tokens (the global
+    layer's positions outgrow the LDS of the wider tiles), against pushes, which
+    attend a token at a time."""
+    tokens = _tokens(8050, seed=12)
+    model = needle3.Model(archive)
+    fed, pushed = model.session(8060), model.session(8060)
+    done = 0
+    for upto in (2200, 4300, 8050):
+        fed.feed(tokens[done:upto])
+        for t in tokens[done:upto]:
+            pushed.push(int(t))
+        done = upto
+        assert np.array_equal(_bits(fed.hidden()), _bits(pushed.hidden())), upto
+        assert np.array_equal(_bits(fed.logits()), _bits(pushed.logits())), upto
+    for layer in range(GEOMETRY["num_layers"]):
+        for a, b in zip(fed.cache(layer), pushed.cache(layer)):
+            assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), layer
+
+
+@pytest.mark.parametrize("scale", [1e-36, 0.0])
+def test_feed_of_values_of_almost_no_magnitude(archive, scale):
+    """Value taps scaled until every value scale is subnormal (weights that a scale
+    of the float's normal range keeps within 12 bits no longer are) or zero."""
+    data = bytearray(archive)
+    a = rn.Archive(data=archive)
+    shape = [GEOMETRY["qkv_conv_taps"], GEOMETRY["num_kv_heads"] * 64]
+    records = [a.record(i) for i in range(a.geometry()["tensor_count"])]
+    taps = [r for r in records if r["kind"] == needle3.KIND_SINGLE and r["shape"] == shape]
+    assert len(taps) == 2 * GEOMETRY["num_layers"]  # k and v of every layer, in turn
+    for r in taps[1::2]:
+        v = np.frombuffer(archive, np.float32, shape[0] * shape[1], r["offset"]) * np.float32(scale)
+        data[r["offset"]:r["offset"] + r["nbytes"]] = v.astype(np.float32).tobytes()
+    data = bytes(data)
+    gs, os_ = needle3.Model(data).session(64), oracle.OracleNeedle3(data).session(64)
+    tokens = _tokens(40, seed=13)
+    gs.feed(tokens)
+    for t in tokens:
+        os_.push(int(t))
+    assert np.array_equal(_bits(gs.hidden()), _bits(os_.hidden()))
+    _compare_session(gs, os_, scale)
