@@ -1342,52 +1342,92 @@ __global__ __launch_bounds__(256) void n3_observe_kernel(const float* cells, N3O
     for (int i = threadIdx.x; i < width; i += blockDim.x) target[i] = target[i] * rescale + weight * cell[i];
 }
 
-// n3_observe_kernel over a run of tokens in order (prefill.rs:92-96): one
-// block per slot; the run's scores first (ops.rs:19-30, 32 tokens at a time,
-// eight lanes each), since they do not depend on the accumulator, then the
-// online updates token by token (heads.rs:138-155).
-__global__ __launch_bounds__(256) void n3_observe_run_kernel(const float* cells, int cell_stride, int count,
-                                                             const float* probes, int k, int width, float* peak,
-                                                             float* total, float* weighted) {
-    __shared__ float score_s[kN3FeedChunk], rescale_s[kN3FeedChunk], weight_s[kN3FeedChunk];
+// n3_observe_kernel over a run of tokens in order (prefill.rs:92-96), in two
+// launches for every slot of every head. What must stay in token order is
+// short: the scores (ops.rs:19-30) do not depend on the accumulator, nor do the
+// running peaks (a maximum, order-free: a prefix maximum of the scores), so
+// every score and every exponential is formed in parallel; the total's and the
+// weighted sums' updates (heads.rs:138-155) follow as chains, one a dimension,
+// over cells requested sixteen tokens ahead. One block a slot with the peaks
+// and exponentials token by token in one thread took 153 us for 256 tokens x 84
+// slots x 768 and a launch a head; these take 21 + 32 us for both heads' 168.
+// scores [slot][kN3FeedChunk + 1]: the run's scores, then the peak before it
+// (which the second launch's blocks read while one of them replaces it).
+__device__ __forceinline__ int n3_slot_head(const N3ObserveHeads& hs) {
+    int hh = 0;
+    for (int j = 1; j < hs.count; ++j) hh = (int)blockIdx.x >= hs.first[j] ? j : hh;
+    return __builtin_amdgcn_readfirstlane(hh);
+}
+
+// 32 tokens a block (blockIdx.y), eight lanes a token
+__global__ __launch_bounds__(256) void n3_observe_scores_kernel(const float* cells, int cell_stride, int count,
+                                                                N3ObserveHeads hs, float* scores) {
     __shared__ float red[256];
-    const int slot = blockIdx.x, layer = slot / k, tid = threadIdx.x;
-    const float* probe = probes + (size_t)slot * width;
-    const float* first_cell = cells + (size_t)layer * width;
-    for (int t0 = 0; t0 < count; t0 += 32) {
-        const int tt = t0 + (tid >> 3), j = tid & 7;
-        if (tt < count) red[tid] = n3_fold<false>(0.0f, first_cell + (size_t)tt * cell_stride + j, probe + j, width / 8, 8);
-        __syncthreads();
-        if (tid < 32 && t0 + tid < count) {
-            const float* cell = first_cell + (size_t)(t0 + tid) * cell_stride;
-            float sum = -0.0f;
-            for (int q = 0; q < 8; ++q) sum = sum + red[8 * tid + q];
-            float tail = -0.0f;
-            for (int i = width / 8 * 8; i < width; ++i) tail = tail + cell[i] * probe[i];
-            score_s[t0 + tid] = (sum + tail) / sqrtf((float)width);
-        }
-        __syncthreads();
-    }
-    if (tid == 0) {
-        float pk = peak[slot], tot = total[slot];
-        for (int t = 0; t < count; ++t) {
-            const float score = score_s[t], next = fmaxf(pk, score);
-            const float rescale = pk == -INFINITY ? 0.0f : libm_expf(pk - next);
-            const float weight = libm_expf(score - next);
-            tot = tot * rescale + weight;
-            pk = next;
-            rescale_s[t] = rescale;
-            weight_s[t] = weight;
-        }
-        peak[slot] = pk;
-        total[slot] = tot;
-    }
+    const int h = n3_slot_head(hs), tid = threadIdx.x, t0 = 32 * blockIdx.y;
+    const int slot = (int)blockIdx.x - hs.first[h], width = hs.width[h];
+    const float* const probe = hs.probes[h] + (size_t)slot * width;
+    const float* const first_cell = cells + (size_t)(slot / hs.k[h]) * width;
+    float* const out = scores + (size_t)blockIdx.x * (kN3FeedChunk + 1);
+    const int tt = min(t0 + (tid >> 3), count - 1), j = tid & 7;
+    red[tid] = n3_fold<false>(0.0f, first_cell + (size_t)tt * cell_stride + j, probe + j, width / 8, 8);
     __syncthreads();
-    float* target = weighted + (size_t)slot * width;
-    for (int i = tid; i < width; i += blockDim.x) {
-        float w = target[i];
-        for (int t = 0; t < count; ++t) w = w * rescale_s[t] + weight_s[t] * first_cell[(size_t)t * cell_stride + i];
-        target[i] = w;
+    if (tid < 32 && t0 + tid < count) {
+        const float* cell = first_cell + (size_t)(t0 + tid) * cell_stride;
+        float sum = -0.0f;
+        for (int q = 0; q < 8; ++q) sum = sum + red[8 * tid + q];
+        float tail = -0.0f;
+        for (int i = width / 8 * 8; i < width; ++i) tail = tail + cell[i] * probe[i];
+        out[t0 + tid] = (sum + tail) / sqrtf((float)width);
+    }
+    if (blockIdx.y == 0 && tid == 0) out[kN3FeedChunk] = hs.peak[h][slot];
+}
+
+// 256 dimensions a block (blockIdx.y); the first also updates the peak and total
+__global__ __launch_bounds__(256) void n3_observe_update_kernel(const float* cells, int cell_stride, int count,
+                                                                N3ObserveHeads hs, const float* scores) {
+    static_assert(kN3FeedChunk == 256, "a token a thread");
+    __shared__ float2 rw_s[kN3FeedChunk];  // rescale, weight
+    __shared__ float wave_s[4];
+    const int h = n3_slot_head(hs), tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int slot = (int)blockIdx.x - hs.first[h], width = hs.width[h];
+    const float* const in = scores + (size_t)blockIdx.x * (kN3FeedChunk + 1);
+    const float old = in[kN3FeedChunk], score = tid < count ? in[tid] : -INFINITY;
+    float next = score;  // the maximum of the scores up to this token
+#pragma unroll
+    for (int m = 1; m < 64; m *= 2) {
+        const float below = __shfl_up(next, m, 64);
+        if (lane >= m) next = fmaxf(next, below);
+    }
+    if (lane == 63) wave_s[wave] = next;
+    const float up = __shfl_up(next, 1, 64);
+    __syncthreads();
+    float before = old;  // the peak before this wave's tokens
+    for (int w = 0; w < wave; ++w) before = fmaxf(before, wave_s[w]);
+    const float previous = lane > 0 ? fmaxf(before, up) : before;
+    next = fmaxf(before, next);
+    rw_s[tid] = make_float2(previous == -INFINITY ? 0.0f : libm_expf(previous - next), libm_expf(score - next));
+    __syncthreads();
+    const int i = 256 * blockIdx.y + tid;
+    const float* const cell = cells + (size_t)(slot / hs.k[h]) * width + min(i, width - 1);
+    float* const target = hs.weighted[h] + (size_t)slot * width + min(i, width - 1);
+    float w = *target;
+    for (int t0 = 0; t0 < count; t0 += 16) {
+        float c[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) c[k] = cell[(size_t)min(t0 + k, count - 1) * cell_stride];
+#pragma unroll
+        for (int k = 0; k < 16; ++k)
+            if (t0 + k < count) {
+                const float2 rw = rw_s[t0 + k];
+                w = w * rw.x + rw.y * c[k];
+            }
+    }
+    if (i < width) *target = w;
+    if (blockIdx.y == 0 && tid == count - 1) {
+        hs.peak[h][slot] = next;
+        float total = hs.total[h][slot];
+        for (int t = 0; t < count; ++t) total = total * rw_s[t].x + rw_s[t].y;
+        hs.total[h][slot] = total;
     }
 }
 
@@ -3215,7 +3255,7 @@ struct rn_n3_session {
         bool ready = false;
         float *stream_a = nullptr, *stream_b = nullptr, *attn = nullptr, *x = nullptr, *input = nullptr;
         float *post = nullptr, *residual = nullptr, *rotated = nullptr, *prod = nullptr, *attended = nullptr;
-        float *qscales = nullptr, *cells = nullptr, *gathered = nullptr, *eraw = nullptr;
+        float *qscales = nullptr, *cells = nullptr, *gathered = nullptr, *eraw = nullptr, *scores = nullptr;
         int8_t* qcodes = nullptr;
         std::vector<float*> ekey, evalue;
     } run;
@@ -3735,16 +3775,6 @@ int enqueue_observe(rn_n3_session* s, const float* cells, int cell_stride, int c
     const rn_n3_model* m = s->m;
     hipStream_t st = s->stream;
     for (size_t b0 = 0; b0 < m->heads.size(); b0 += kN3MaxHeads) {
-        if (count > 1) {
-            for (size_t i = b0; i < std::min(m->heads.size(), b0 + kN3MaxHeads); ++i) {
-                const N3Head& h = m->heads[i];
-                rn_launch(n3_observe_run_kernel, dim3(h.layers * h.per_layer), dim3(256), 0, st, cells, cell_stride,
-                          count, (const float*)h.probes, h.per_layer, h.width, s->peak[i], s->total[i],
-                          s->weighted[i]);
-                N3_HIP(hipGetLastError());
-            }
-            continue;
-        }
         N3ObserveHeads hs{};
         int blocks = 0;
         for (size_t i = b0; i < std::min(m->heads.size(), b0 + kN3MaxHeads); ++i) {
@@ -3760,7 +3790,16 @@ int enqueue_observe(rn_n3_session* s, const float* cells, int cell_stride, int c
             blocks += h.layers * h.per_layer;
         }
         hs.first[hs.count] = blocks;
-        rn_launch(n3_observe_kernel, dim3(blocks), dim3(256), 0, st, cells, hs);
+        if (count > 1) {
+            const int widest = *std::max_element(hs.width, hs.width + hs.count);
+            rn_launch(n3_observe_scores_kernel, dim3(blocks, (count + 31) / 32), dim3(256), 0, st, cells, cell_stride,
+                      count, hs, s->run.scores);
+            N3_HIP(hipGetLastError());
+            rn_launch(n3_observe_update_kernel, dim3(blocks, (widest + 255) / 256), dim3(256), 0, st, cells, cell_stride,
+                      count, hs, (const float*)s->run.scores);
+        } else {
+            rn_launch(n3_observe_kernel, dim3(blocks), dim3(256), 0, st, cells, hs);
+        }
         N3_HIP(hipGetLastError());
     }
     return RN_OK;
@@ -3852,6 +3891,9 @@ int run_buffers(rn_n3_session* s) {
     N3_CALL(alloc_n(s, C * (A + 1) * d, &r.cells));
     N3_CALL(alloc_n(s, C * gathered, &r.gathered));
     N3_CALL(alloc_n(s, C * d, &r.eraw));
+    size_t slots = 1;
+    for (const N3Head& h : m->heads) slots += (size_t)h.layers * h.per_layer;
+    N3_CALL(alloc_n(s, slots * (C + 1), &r.scores));
     r.ekey.assign(g.engram_site_count, nullptr);
     r.evalue.assign(g.engram_site_count, nullptr);
     for (uint32_t e = 0; e < g.engram_site_count; ++e) {

@@ -280,6 +280,8 @@ def test_long_feed_equals_pushes(archive):
         done = upto
         assert np.array_equal(_bits(fed.hidden()), _bits(pushed.hidden())), upto
         assert np.array_equal(_bits(fed.logits()), _bits(pushed.logits())), upto
+        for code in (1, 2):  # the probe heads, over whole runs of 256 tokens and a shorter last one
+            assert np.array_equal(_bits(fed.pooled_readout(code)), _bits(pushed.pooled_readout(code))), (upto, code)
     for layer in range(GEOMETRY["num_layers"]):
         for a, b in zip(fed.cache(layer), pushed.cache(layer)):
             assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), layer
