@@ -21,6 +21,8 @@
 //   total and P.V (T3): thirty-two running sums over positions j, j+32, ... in
 //               increasing order, then added j = 0..31.
 // Scores live in LDS (dynamic, one float per position).
+#include <type_traits>
+
 #include "rn_device.hpp"
 #include "rn_internal.hpp"
 
@@ -33,6 +35,7 @@ constexpr int kClasses = 32;  // T3 position classes (p mod 32)
 template <int DPV> struct ValuePiece;
 template <> struct ValuePiece<8> { using T = uint4; };
 template <> struct ValuePiece<4> { using T = uint2; };
+template <> struct ValuePiece<2> { using T = uint32_t; };
 template <int DPV>
 __device__ __forceinline__ void unpack_values(const typename ValuePiece<DPV>::T& raw, float* out) {
     const __half2* h = reinterpret_cast<const __half2*>(&raw);
@@ -351,7 +354,7 @@ hipError_t launch_attend(const AttendParams& p, int mode, int grid_x, int grid_y
 
 // Causal prefill attention over query tiles: one 256-thread block per (head,
 // QT consecutive queries), so each key and value row is read from L2 once per
-// tile instead of once per query. Rows go to LDS in chunks of 256 positions
+// tile instead of once per query. Rows go to LDS in chunks
 // (global_load_lds: no registers); the scores of the QT queries live in LDS
 // [QT][length]. The float order is the per-query kernel's: scores in tree T2
 // (4 lanes per key row, the row's 16 dims per lane reused for all QT
@@ -361,18 +364,22 @@ hipError_t launch_attend(const AttendParams& p, int mode, int grid_x, int grid_y
 typedef __attribute__((address_space(3))) void lds_void;
 typedef __attribute__((address_space(1))) void global_void;
 
-constexpr int kTileRows = 256;  // positions per staged chunk
-
-template <int QT>
-__global__ __launch_bounds__(256) void attend_prefill_tile_kernel(AttendParams p, int count) {
+// ROWS positions per staged chunk. A context that one 256-row chunk holds is
+// staged once; longer ones take 128-row chunks, half the LDS, so that twice the
+// blocks share a CU: a lone wave a SIMD issues a vector instruction every 5.5
+// cycles, two or more every 2.7 (adds, multiplies) to 4.5 (fp16 products) between
+// them (1000 tokens x 8 heads: 98 us with 256-row chunks, 49 with 128; 256
+// tokens: 9.1 and 9.9).
+template <int QT, int ROWS>
+__global__ __launch_bounds__(256) void attend_prefill_kernel(AttendParams p, int count) {
     constexpr int NT = 256;
     extern __shared__ float scores[];  // [QT][max length]
-    __shared__ __align__(16) __half k_s[kTileRows * kHeadDim];  // a chunk of key rows
-    __shared__ __align__(16) __half v_s[kTileRows * kHeadDim];  // a chunk of value rows
+    __shared__ __align__(16) __half kv_s[2][ROWS * kHeadDim];  // a chunk of key rows, one of value rows
+    __half *const k_s = kv_s[0], *const v_s = kv_s[1];
     __shared__ float q_s[QT][kHeadDim];
     __shared__ float total_s[QT][kClasses];
-    float(*part_s)[kClasses][kHeadDim] = reinterpret_cast<float(*)[kClasses][kHeadDim]>(k_s);
-    static_assert(QT * kClasses * kHeadDim * 4 <= kTileRows * kHeadDim * 2, "class sums fit in the key buffer");
+    float(*part_s)[kClasses][kHeadDim] = reinterpret_cast<float(*)[kClasses][kHeadDim]>(kv_s);
+    static_assert(QT * kClasses * kHeadDim * 4 <= 2 * ROWS * kHeadDim * 2, "class sums fit in the chunks");
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     // the last tiles attend the most positions: they go first
@@ -386,10 +393,10 @@ __global__ __launch_bounds__(256) void attend_prefill_tile_kernel(AttendParams p
     for (int q = 0; q < QT; ++q) len[q] = t0 + q < count ? p.first + t0 + q + 1 : 0;
     const int L = p.first + min(t0 + QT, count);  // rows the tile needs (t0 < count)
 
-    // a chunk of rows [c0, c0 + 256) of K or V into dst; rows past L repeat row L - 1
+    // a chunk of rows [c0, c0 + ROWS) of K or V into dst; rows past L repeat row L - 1
     auto stage = [&](const __half* src, __half* dst, int c0) {
 #pragma unroll
-        for (int i = 0; i < kTileRows * 8 / NT; ++i) {
+        for (int i = 0; i < ROWS * 8 / NT; ++i) {
             const int piece = NT * i + 64 * wave + lane, row = min(c0 + piece / 8, L - 1);
             __builtin_amdgcn_global_load_lds((global_void*)(src + (size_t)row * kHeadDim + 8 * (piece % 8)),
                                              (lds_void*)(dst + 8 * (NT * i + 64 * wave)), 16, 0, 0);
@@ -407,7 +414,7 @@ __global__ __launch_bounds__(256) void attend_prefill_tile_kernel(AttendParams p
     const int r = tid >> 2, li = tid & 3;
     const float inverse_root = 1.0f / sqrtf((float)kHeadDim);
     float qr[QT][16];  // this lane's 16 query dims of every query
-    for (int c0 = 0; c0 < L; c0 += kTileRows) {
+    for (int c0 = 0; c0 < L; c0 += ROWS) {
         if (c0 > 0) {
             __syncthreads();  // the previous chunk is consumed
             stage(K, k_s, c0);
@@ -420,7 +427,7 @@ __global__ __launch_bounds__(256) void attend_prefill_tile_kernel(AttendParams p
 #pragma unroll
                 for (int i = 0; i < 16; ++i) qr[q][i] = q_s[q][16 * li + i];
         }
-        for (int pass = 0; pass < kTileRows && c0 + pass < L; pass += NT / 4) {
+        for (int pass = 0; pass < ROWS && c0 + pass < L; pass += NT / 4) {
             const int pp = c0 + pass + r;
             const uint4* kr = reinterpret_cast<const uint4*>(k_s + (pass + r) * kHeadDim + 16 * li);
             const uint4 ka = kr[0], kb = kr[1];
@@ -453,7 +460,7 @@ __global__ __launch_bounds__(256) void attend_prefill_tile_kernel(AttendParams p
 #pragma unroll
         for (int i = 0; i < 8; ++i) acc[q][i] = 0.0f;
     }
-    for (int c0 = 0; c0 < L; c0 += kTileRows) {
+    for (int c0 = 0; c0 < L; c0 += ROWS) {
         __syncthreads();  // weights written; the previous chunk is consumed
         if (c0 > 0) {
             stage(V, v_s, c0);
@@ -461,7 +468,7 @@ __global__ __launch_bounds__(256) void attend_prefill_tile_kernel(AttendParams p
             __syncthreads();
         }
         // positions every query of the tile attends, then the tile's last QT - 1
-        const int all = min(c0 + kTileRows, len[0]), end = min(c0 + kTileRows, L);
+        const int all = min(c0 + ROWS, len[0]), end = min(c0 + ROWS, L);
         int pp = c0 + j;
         // e times the fp16 value by v_fma_mix_f32 (the exact product rounded once)
         auto weigh = [&](float (&a)[8], float e, const uint4& raw) {
@@ -491,7 +498,7 @@ __global__ __launch_bounds__(256) void attend_prefill_tile_kernel(AttendParams p
             }
         }
     }
-    // the key buffer becomes the class sums (its last readers passed the barrier above)
+    __syncthreads();  // the chunks become the class sums
 #pragma unroll
     for (int q = 0; q < QT; ++q) {
 #pragma unroll
@@ -514,18 +521,231 @@ __global__ __launch_bounds__(256) void attend_prefill_tile_kernel(AttendParams p
     }
 }
 
-// The tiled kernel holds the scores of QT queries over the whole length in LDS;
-// longer contexts take the per-query kernel.
-constexpr int kPrefillTileQueries = 4;
-constexpr int kPrefillTileMaxLength = 6144;
+constexpr int kPrefillTileQueries = 16;
 
+// Causal prefill attention on the f32 matrix instructions: one 1024-thread block
+// per (head, 16 consecutive queries).
+//
+// The float order is the per-query kernels': scores in tree T2, fast_exp weights,
+// value sums in T3, each product rounded before its addition. A fused
+// multiply-add would round once, so no accumulator carries a sum here: every
+// v_mfma_f32_16x16x1_4b adds one product to +0, which rounds it exactly as the
+// vector multiply does (equal on all inputs tried, subnormal, infinite and NaN
+// ones included, but for the sign of a zero, which no later addition sees: the
+// running sums start at +0 and are never -0), and the vector unit only adds.
+// The matrix pipe forms 32 products a cycle beside the vector unit's 16 adds.
+// Its four blocks are four independent outer products of 16 queries:
+//   1. scores: block b takes sub-sum 4 m + b of the T2 tree, in step (m, i) its
+//      dimension i, against 16 keys; the sub-sums' adds and the tree run on the
+//      result registers (lane (g, c): queries 4 g + i, key c).
+//   2. peaks and weights, a wave a row, then the class totals, a thread a
+//      (query, class) chain.
+//   3. values: a wave serves four position classes and half the dimensions; block b
+//      takes class 4 c + b at step s (position 32 s + 4 c + b) against 16
+//      dimensions, so the classes' running sums stay in registers and walk the
+//      positions in order.
+//   4. the class groups add to the sums of those before them, in order, through
+//      4 KB of LDS.
+// Bound by the products and additions: 10.4 SIMD cycles a (query, position) pair
+// (2.25 a 64 products, 2.9 a 64 adds; a fp16 product on the vector unit takes
+// 4.5), 17 us for 1000 tokens x 8 heads; measured 40 us a launch with the phases'
+// latencies, against 98 with four queries a block on the vector unit.
+__global__ __launch_bounds__(1024) void attend_prefill_tile_kernel(AttendParams p, int count, int pitch) {
+    typedef float v16f __attribute__((ext_vector_type(16)));
+    constexpr int NW = 16, QT = kPrefillTileQueries, DT = 2;  // waves; queries; dimensions a lane sums per class
+    extern __shared__ __align__(16) float scores[];  // [16][pitch]
+    __shared__ float total_s[16][kClasses + 1], inverse_s[16];
+    __shared__ __align__(8) float sum_s[2][16][32];  // the classes added so far, [half][query][2 c + d]
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int g = lane >> 4, c16 = lane & 15;
+    // the last tiles attend the most positions: they go first
+    const int h = blockIdx.x, t0 = (gridDim.y - 1 - blockIdx.y) * QT, live = min(QT, count - t0);
+    const size_t base = ((size_t)p.layer * p.heads + h) * p.capacity * kHeadDim;
+    const __half* const K = p.kc + base;
+    const __half* const V = p.vc + base;
+    const int len0 = p.first + t0 + 1, L = p.first + t0 + live;  // query t attends len0 + t positions
+    const int row = min(c16, live - 1);                // this lane's query as an operand row
+    const v16f zero = {};
+    // (an operand of the product after next, held back until this step's sums are
+    // formed: left free, the compiler issues every product first and spills them)
+    auto hold = [](v16f& sums, float& operand) { asm volatile("" : "+v"(sums), "+v"(operand)); };
+    auto product = [&](float a, float b) { return __builtin_amdgcn_mfma_f32_16x16x1f32(a, b, zero, 0, 0, 0); };
+
+    // 1. scores (T2)
+    float qa[16];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+        const float4 f = *reinterpret_cast<const float4*>(p.q + (size_t)(t0 + row) * p.d_model + h * kHeadDim + 16 * m + 4 * g);
+        qa[4 * m] = f.x;
+        qa[4 * m + 1] = f.y;
+        qa[4 * m + 2] = f.z;
+        qa[4 * m + 3] = f.w;
+    }
+    const float inverse_root = 1.0f / sqrtf((float)kHeadDim);
+    auto load_keys = [&](int n0, uint2 (&k)[4]) {
+        const __half* src = K + (size_t)min(n0 + c16, L - 1) * kHeadDim + 4 * g;
+#pragma unroll
+        for (int m = 0; m < 4; ++m) k[m] = *reinterpret_cast<const uint2*>(src + 16 * m);
+    };
+    uint2 kr[4];
+    load_keys(16 * wave, kr);
+    for (int n0 = 16 * wave; n0 < L; n0 += 16 * NW) {
+        float part[4][4], kf[16];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) unpack_values<4>(kr[m], kf + 4 * m);
+        load_keys(n0 + 16 * NW, kr);
+        // the products of step k + 1 form while those of step k are added
+        v16f pr = product(qa[0], kf[0]), s = zero;
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+            const v16f d = pr;
+            if (k + 1 < 16) pr = product(qa[k + 1], kf[k + 1]);
+            s = k % 4 == 0 ? d : s + d;
+            hold(s, kf[min(k + 2, 15)]);
+            if (k % 4 == 3)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) part[k / 4][i] = (s[i] + s[4 + i]) + (s[8 + i] + s[12 + i]);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float sc = (part[0][i] + part[1][i]) + (part[2][i] + part[3][i]);
+            scores[(size_t)(4 * g + i) * pitch + n0 + c16] = sc * inverse_root;
+        }
+    }
+    // the first value rows, requested under the weights
+    const int cg = wave >> 1, half = wave & 1;  // class group, dimension half
+    using VPiece = typename ValuePiece<DT>::T;
+    constexpr int PB = 4;  // steps of values in flight
+    auto load_values = [&](int s0, VPiece (&v)[PB]) {
+#pragma unroll
+        for (int k = 0; k < PB; ++k)
+            v[k] = *reinterpret_cast<const VPiece*>(V + (size_t)min(kClasses * (s0 + k) + 4 * cg + g, L - 1) * kHeadDim +
+                                                    4 * c16 + 2 * half);
+    };
+    VPiece vr[PB];
+    load_values(0, vr);
+    __syncthreads();
+
+    // 2. peak (order-free) and the fast_exp weights, then the class totals
+    for (int q = wave; q < live; q += NW) {
+        float* const sc = scores + (size_t)q * pitch;
+        const int n = len0 + q;
+        float m = -INFINITY;
+        for (int pp = lane; pp < n; pp += 64) m = fmaxf(m, sc[pp]);
+        m = wave_max(m);
+        for (int pp = lane; pp < n; pp += 64) sc[pp] = fast_exp(sc[pp] - m);
+    }
+    __syncthreads();
+    if (tid < 16 * kClasses) {
+        const int q = tid / kClasses, j = tid % kClasses;
+        if (q < live) {
+            const float* const sc = scores + (size_t)q * pitch;
+            const int n = len0 + q;
+            float t = 0.0f;
+            int pp = j;
+            for (; pp + 7 * kClasses < n; pp += 8 * kClasses) {
+                float e[8];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) e[k] = sc[pp + k * kClasses];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) t = t + e[k];
+            }
+            for (; pp < n; pp += kClasses) t = t + sc[pp];
+            total_s[q][j] = t;
+        }
+    }
+
+    // 3. weighted values (T3)
+    lds_barrier();  // the totals, for step 4
+    v16f acc[DT] = {zero, zero};  // [dimension][4 b + i]: class 4 cg + b, query 4 g + i
+    const float* const e_s = scores + (size_t)c16 * pitch + 4 * cg + g;
+    // one step, the products of the next dimension under the current one's additions
+    auto step = [&](auto masked, int s, const VPiece& raw) {
+        const float e = e_s[kClasses * s];
+        float v[DT];
+        unpack_values<DT>(raw, v);
+        v16f pr = product(e, v[0]);
+#pragma unroll
+        for (int d = 0; d < DT; ++d) {
+            const v16f now = pr;
+            if (d + 1 < DT) pr = product(e, v[d + 1]);
+            const v16f t = acc[d] + now;
+            if constexpr (decltype(masked)::value) {
+#pragma unroll
+                for (int m = 0; m < 16; ++m)
+                    acc[d][m] = kClasses * s + 4 * cg + m / 4 < len0 + 4 * g + m % 4 ? t[m] : acc[d][m];
+            } else {
+                acc[d] = t;
+            }
+            hold(acc[d], v[min(d + 2, DT - 1)]);
+        }
+    };
+    const int steps = (L + kClasses - 1) / kClasses, plain = len0 / kClasses;  // every query attends all of the first
+    for (int s0 = 0; s0 < steps; s0 += PB) {
+        VPiece vn[PB];
+        load_values(s0 + PB, vn);
+        if (s0 + PB <= plain) {
+#pragma unroll
+            for (int k = 0; k < PB; ++k) step(std::false_type(), s0 + k, vr[k]);
+        } else {
+#pragma unroll
+            for (int k = 0; k < PB; ++k) {
+                if (s0 + k < plain) step(std::false_type(), s0 + k, vr[k]);
+                else if (s0 + k < steps) step(std::true_type(), s0 + k, vr[k]);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < PB; ++k) vr[k] = vn[k];
+    }
+
+    // 4. the classes in order: each group adds its four to the sums of those before it
+    for (int w = 0; w < kClasses / 4; ++w) {
+        if (w == cg) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float2* const slot = reinterpret_cast<float2*>(&sum_s[half][4 * g + i][2 * c16]);
+                float2 o = w == 0 ? make_float2(0.0f, 0.0f) : *slot;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    o.x = o.x + acc[0][4 * k + i];
+                    o.y = o.y + acc[1][4 * k + i];
+                }
+                *slot = o;
+            }
+        } else if (w == 0 && wave == NW - 1 && lane < live) {  // the last wave waits longest
+            float t = 0.0f;
+#pragma unroll
+            for (int k = 0; k < kClasses; ++k) t = t + total_s[lane][k];
+            inverse_s[lane] = reciprocal(t);
+        }
+        lds_barrier();
+    }
+    const int r = tid >> 9, q = (tid >> 5) & 15, d = tid & 31;
+    if (q < live)
+        p.out[(size_t)(t0 + q) * p.d_model + h * kHeadDim + 4 * (d >> 1) + 2 * r + (d & 1)] = sum_s[r][q][d] * inverse_s[q];
+}
+
+// The matrix tiles for at least 640 tokens (512 blocks of 16 queries would leave
+// a CU idle before that; 500 tokens 20.2 against 19.8 us, 1000 tokens 40 against 49)
+// while 16 score rows fit the LDS (2300 positions); rows 4 floats past a
+// multiple of 128 hold whole steps and start an operand read's 16 rows on distinct
+// banks. Otherwise four queries a block, and past 6144 positions the per-query
+// kernel.
 hipError_t launch_attend_prefill(const AttendParams& p, int heads, int count, hipStream_t stream) {
     if (count <= 0) return hipSuccess;
-    const int length = p.first + count;
-    if (length > kPrefillTileMaxLength) return launch_attend(p, kAttendPrefill, heads, count, length, stream);
-    const size_t lds = sizeof(float) * (size_t)kPrefillTileQueries * length;
-    const dim3 grid(heads, (count + kPrefillTileQueries - 1) / kPrefillTileQueries);
-    rn_launch(attend_prefill_tile_kernel<kPrefillTileQueries>, grid, dim3(256), lds, stream, p, count);
+    constexpr int QT = 4, kMaxLength = 6144;
+    const int length = p.first + count, pitch = (length + 127) / 128 * 128 + 4;
+    const size_t tile_lds = sizeof(float) * kPrefillTileQueries * (size_t)pitch, lds = sizeof(float) * QT * (size_t)length;
+    const dim3 grid(heads, (count + QT - 1) / QT);
+    if (count >= 640 && tile_lds <= 148 * 1024)
+        rn_launch(attend_prefill_tile_kernel, dim3(heads, (count + kPrefillTileQueries - 1) / kPrefillTileQueries), dim3(1024),
+                  tile_lds, stream, p, count, pitch);
+    else if (length > kMaxLength)
+        return launch_attend(p, kAttendPrefill, heads, count, length, stream);
+    else if (length <= 256)
+        rn_launch((attend_prefill_kernel<QT, 256>), grid, dim3(256), lds, stream, p, count);
+    else
+        rn_launch((attend_prefill_kernel<QT, 128>), grid, dim3(256), lds, stream, p, count);
     return hipGetLastError();
 }
 

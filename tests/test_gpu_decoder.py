@@ -153,6 +153,35 @@ def test_feed_small_and_ragged_counts(tiny, count):
     assert np.array_equal(_bits(gs.logits()), _bits(os_.logits()))
 
 
+@pytest.mark.parametrize("cached,count", [
+    (0, 300),      # past the 256 rows one staged chunk holds
+    (0, 640),      # whole 16-query tiles on the matrix instructions
+    (37, 701),     # a ragged last tile behind a cached prefix
+    (1600, 645),   # the longest context of the tiles
+    (1690, 660),   # the first past it
+])
+def test_long_feed_bit_exact(tiny_config, tiny_weights, cached, count):
+    cfg = dict(tiny_config, max_positions=2400)
+    gs = rn.Model(cfg, tiny_weights).session(cached + count)
+    os_ = oracle.OracleModel(cfg, tiny_weights).session(cached + count)
+    if cached:
+        k, v = rn.synthetic_cache(cfg, cached, "longfeed")
+        gs.set_cache(k, v)
+        os_.set_cache(k, v)
+    tokens = rn.synth_tokens(rn.SEED, "longfeed.tokens", cfg["vocab"], count)
+    oracle.set_threads(8)
+    try:
+        gs.feed(tokens)
+        os_.feed(tokens)
+        assert np.array_equal(_bits(gs.hidden()), _bits(os_.hidden))
+        assert np.array_equal(_bits(gs.logits()), _bits(os_.logits()))
+    finally:
+        oracle.set_threads(1)
+    gk, gv = gs.get_cache()
+    assert np.array_equal(gk.view(np.uint16), os_.keys[:, :, :cached + count])
+    assert np.array_equal(gv.view(np.uint16), os_.values[:, :, :cached + count])
+
+
 def test_clone_is_independent(tiny, tiny_config):
     gm, _ = tiny
     k, v = rn.synthetic_cache(tiny_config, 10, "clone")
