@@ -138,7 +138,13 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT >= 512 ? 
             nv[1] = row[2 * p.d_model + kHeadDim / 2];
         }
     }
-    if constexpr (POS_FIRST) {
+    if constexpr (MODE == kAttendRaw && POS_FIRST) {
+        rows = p.lengths[blockIdx.x];
+        if (rows < 1 || rows > p.stride) {
+            if (tid == 0) *p.error = 4;
+            return;
+        }
+    } else if constexpr (POS_FIRST) {
         pos = p.pos[(size_t)blockIdx.y * p.pos_stride];
         if (pos < 0 || pos >= p.capacity) {
             if (tid == 0) atomicOr(p.error, 2);
@@ -215,10 +221,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT >= 512 ? 
         has_new = false;
         if (tid < kHeadDim) q_s[tid] = p.q[(size_t)blockIdx.y * p.d_model + blockIdx.x * kHeadDim + tid];
     } else {
-        nglobal = p.lengths[blockIdx.x];
+        nglobal = POS_FIRST ? rows : p.lengths[blockIdx.x];
         has_new = false;
         if (nglobal < 1 || nglobal > p.stride) {
-            if (tid == 0) atomicOr(p.error, 4);
+            if (tid == 0) *p.error = 4;  // (host memory: stores of one value, no atomic)
             return;
         }
         if (tid < kHeadDim) q_s[tid] = p.q[(size_t)blockIdx.x * kHeadDim + tid];
@@ -335,16 +341,34 @@ hipError_t launch_attend(const AttendParams& p, int mode, int grid_x, int grid_y
     const dim3 grid(grid_x, grid_y);
     switch (mode) {
         case kAttendDecode:
-            if (grid_y == 1)  // one sequence: its loads go out before its position is read
+            // one sequence: its loads go out before its position is read. Many ragged
+            // ones clamp their loads to their own positions: while the blocks do not
+            // fill the chip, passes of 384 keys and 288 values (20 sequences of up to
+            // 700: 718 us a step against 740 with 640 and 576); once they do, short
+            // caches take 256-thread blocks, four a CU (96 sequences of up to 60: 691
+            // against 792), long ones a single pass up to 576 positions (64 of up to
+            // 512: 782 us a step, 812 in 256-position passes).
+            if (grid_y == 1)
                 rn_launch((attend_kernel<kAttendDecode, 6, 12, false>), grid, dim3(256), lds, stream, p);
-            else              // many ragged sequences: exact clamps, one pass up to 576 positions
+            else if (grid_x * grid_y < 256)
+                rn_launch((attend_kernel<kAttendDecode, 3, 9, true, 512>), grid, dim3(512), lds, stream, p);
+            else if (max_length <= 256)
+                rn_launch((attend_kernel<kAttendDecode, 4, 8, true>), grid, dim3(256), lds, stream, p);
+            else
                 rn_launch((attend_kernel<kAttendDecode, 5, 18, true, 512>), grid, dim3(512), lds, stream, p);
             break;
         case kAttendPrefill:
             rn_launch((attend_kernel<kAttendPrefill, 4, 8, false>), grid, dim3(256), lds, stream, p);
             break;
         case kAttendRaw:
-            rn_launch((attend_kernel<kAttendRaw, 6, 12, false>), grid, dim3(256), lds, stream, p);
+            // the length first: a ragged problem's blocks fetch its own rows only, in
+            // short passes whose registers leave four blocks a CU (512 heads of up to 512
+            // positions 20.1 us a call against 25.3 with the rows requested before the
+            // length); a few long ones take 512 threads (4 x 4000: 27.1 against 30.6)
+            if (grid_x <= 64 && p.stride > 768)
+                rn_launch((attend_kernel<kAttendRaw, 5, 18, true, 512>), grid, dim3(512), lds, stream, p);
+            else
+                rn_launch((attend_kernel<kAttendRaw, 4, 8, true>), grid, dim3(256), lds, stream, p);
             break;
         default:
             return hipErrorInvalidValue;

@@ -239,6 +239,26 @@ def test_batch_decode_equals_sessions_and_oracle(tiny, tiny_config):
             assert ids[i].tolist() == o.greedy(int(first[i]), steps).tolist(), i
 
 
+@pytest.mark.parametrize("heads_blocks,capacity", [(300, 250), (300, 300)])
+def test_batch_decode_with_a_full_chip(tiny, tiny_config, heads_blocks, capacity):
+    """More than 256 attention blocks, with caches of one 256-position pass and past it."""
+    gm, _ = tiny
+    count, steps = -(-heads_blocks // tiny_config["heads"]), 4
+    lengths = rn.synth_tokens(rn.SEED, "full.lengths", capacity - steps, count) + 1
+    lengths[0] = capacity - steps
+    first = rn.synth_tokens(rn.SEED, "full.first", tiny_config["vocab"], count)
+    k, v = rn.synthetic_cache(tiny_config, capacity, "full")
+    b = rn.Batch(gm, count, capacity)
+    for i, n in enumerate(lengths):
+        b.set_cache(i, np.ascontiguousarray(k[:, :, :n]), np.ascontiguousarray(v[:, :, :n]))
+    ids = b.decode_greedy(first, steps)
+    for i in (0, 1, count // 2, count - 1):
+        s = gm.session(capacity)
+        s.set_cache(np.ascontiguousarray(k[:, :, :lengths[i]]), np.ascontiguousarray(v[:, :, :lengths[i]]))
+        assert ids[i].tolist() == s.decode_greedy(int(first[i]), steps).tolist(), i
+        assert np.array_equal(_bits(b.logits()[i]), _bits(s.logits())), i
+
+
 def test_full_decode_workload_bit_identical():
     """The batch-1 decode workload at full size: 20 layers, d 512, vocab 8192,
     fp16 cache pre-filled to 256, 64 greedy tokens — ids equal the oracle's."""

@@ -182,6 +182,23 @@ def test_attend_heads_bit_exact(lengths):
         assert np.array_equal(out[i].view(np.uint32), ref.view(np.uint32)), (i, L)
 
 
+@pytest.mark.parametrize("count,stride", [
+    (70, 600),    # 256-thread blocks: lengths around their passes of 256 positions
+    (64, 769),    # few long problems: 512-thread blocks
+    (3, 1300),    # and past their passes of 640 keys and 576 values
+])
+def test_attend_heads_of_many_lengths(count, stride):
+    edges = [1, 2, 31, 32, 33, 64, 255, 256, 257, 288, 511, 512, 513, 575, 576, 577, 640, 641, 1153, 1281]
+    lengths = np.array([stride] + [min(edges[i % len(edges)], stride) for i in range(1, count)], np.int32)
+    q = rn.synth_normal(7, "attend.q", 1.0, (count, 64))
+    K = rn.synth_normal_f16(7, "attend.k", (count, stride, 64))
+    V = rn.synth_normal_f16(7, "attend.v", (count, stride, 64))
+    out = rn.attend_heads(q, K, V, lengths)
+    for i, n in enumerate(lengths):
+        ref = oracle.attend_head(q[i], K[i, :n], V[i, :n])
+        assert np.array_equal(out[i].view(np.uint32), ref.view(np.uint32)), (i, n)
+
+
 def test_attend_heads_rejects_bad_length():
     q = np.zeros((1, 64), np.float32)
     K = np.zeros((1, 4, 64), np.float16)
