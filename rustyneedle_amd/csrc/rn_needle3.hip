@@ -576,7 +576,7 @@ struct N3QkvParams {
 // rotary for q and k, int8 codes per head, the cache append. One wave per head
 // (blocks 0..H-1 the queries, then the key and value heads) and token
 // (blockIdx.y: position + t; attention.rs:242-318 for a run of tokens, whose
-// raw rows join the ring afterwards, n3_ring_store_kernel).
+// raw rows join the ring afterwards, in the attention launch).
 __global__ __launch_bounds__(64) void n3_qkv_kernel(N3QkvParams p) {
     __shared__ float v_s[kN3Head];
     __shared__ float red[8];
@@ -658,6 +658,11 @@ struct N3AttendParams {
     float inverse_root;
     float* out;            // [H][64]
     int gate_stride;       // a run of tokens: token t's gates at gate + t * gate_stride
+    // a run: its last min(count, ring_keep) raw q | k | v rows join the conv-tap
+    // ring [ring_keep][ring_width] here, after every tap of the run has been read
+    const float* ring_rows;  // gate_stride apart
+    float* ring;
+    int ring_keep, ring_width;
 };
 
 // kernels/src/attention.rs:53-80 for query head blockIdx.x of the token at
@@ -802,6 +807,14 @@ __global__ __launch_bounds__(kN3TileThreads) void n3_attend_tile_kernel(N3Attend
         v = fmaxf(v, __int_as_float(dpp_move<0x141>(__float_as_int(v))));
         return fmaxf(v, __int_as_float(dpp_move<0x140>(__float_as_int(v))));
     };
+
+    if (blockIdx.y == 0 && p.ring_keep > 0) {  // as n3_ring_store_kernel; a slice of the width a head
+        const int n = min(count, p.ring_keep);
+        for (int i = h * kN3TileThreads + tid; i < n * p.ring_width; i += H * kN3TileThreads) {
+            const int t = count - n + i / p.ring_width, c = i % p.ring_width;
+            p.ring[(size_t)((p.position + t) % p.ring_keep) * p.ring_width + c] = p.ring_rows[(size_t)t * p.gate_stride + c];
+        }
+    }
 
     // 1. this lane's tokens are 4 q + i, its positions n + r16
     const v4i aq = *reinterpret_cast<const v4i*>(p.qcodes + ((size_t)(t0 + min(r16, live - 1)) * H + h) * kN3Head + 16 * q);
@@ -4042,13 +4055,9 @@ int enqueue_run(rn_n3_session* s, const uint32_t* tokens, int count) {
         qp.run = 1;
         rn_launch(n3_qkv_kernel, dim3(H + 2 * KV, T), dim3(64), 0, st, qp);
         N3_HIP(hipGetLastError());
-        if (qp.ntaps > 0) {
-            rn_launch(n3_ring_store_kernel, dim3((qkv + 255) / 256, std::min(T, qp.ntaps)), dim3(256), 0, st,
-                      (const float*)r.prod, rows, T, P0, qp.ntaps, qkv, c.hist, qkv);
-            N3_HIP(hipGetLastError());
-        }
         N3AttendParams ap{r.qcodes, r.qscales, c.keys, c.key_scales, c.values, c.value_scales, r.prod + qkv,
-                          s->capacity, P0, layer_window(g, layer), H / KV, 1.0f / sqrtf(64.0f), r.attended, rows};
+                          s->capacity, P0, layer_window(g, layer), H / KV, 1.0f / sqrtf(64.0f), r.attended, rows,
+                          r.prod, c.hist, qp.ntaps, qkv};
         // 16 tokens a block, fewer where their rows would not fit the LDS; rows
         // 4 floats past a multiple of 64, so that neighbours start on other banks
         int tile = 16, pitch = 0;
