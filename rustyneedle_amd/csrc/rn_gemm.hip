@@ -283,6 +283,8 @@ __global__ __launch_bounds__(1024) void gemm_split_kernel(GemmParams p) {
 }
 
 // ---- the chain GEMM: group chains kept in the MFMA result registers ----------
+// (the form that also writes the int32 sums out; products without them take the
+// panel and ring forms below)
 //
 // A 256-thread block (4 waves, WAVES_M x (4 / WAVES_M)) owns a BM x BN output
 // tile; each wave owns SM x SN sub-tiles of 16 x 16, and each lane 4 outputs per
@@ -694,6 +696,206 @@ __global__ __launch_bounds__(256) void gemm_panel_kernel(GemmParams p) {
         }
 }
 
+// ---- the ring GEMM: K chunks through a ring of LDS images ------------------------
+//
+// The panel kernel's chunk images (128 columns of the tile's rows, 16-byte
+// pieces XOR-swizzled by the row, filled by global_load_lds) in a ring of S, for
+// any K of whole chunks and tiles that keep more rows than a whole K panel
+// would fit: while a chunk's groups are folded, the next S - 2 are in flight, so
+// neither the width of a row nor the tile sets how often a block waits for
+// memory. Chunk c + S - 1 is requested into the image that chunk c - 1 left, after
+// the barrier that shows every wave done with it. The tile's weight scales are
+// loaded whole, first.
+// The group sums leave the matrix core as the bit pattern of a float: the
+// accumulator starts at the bits of 1.5 2^23, so the int32 sum (below 2^20 in
+// magnitude) lands in its mantissa, and one subtraction (2.9 SIMD cycles; a
+// conversion takes 4.3) gives the exact float.
+// Bound by the epilogue's vector work (10 SIMD cycles a 64 sums, the rest of a
+// group's 20 its operand reads) with the loads hidden: 2048 x 8192 x 2048 in 155
+// us, 444 TOPS, with the quantisation, where chunks double-buffered through
+// registers took 200.
+constexpr float kSumBias = 12582912.0f;  // 1.5 2^23
+
+template <int SM, int SN, int WM, int WN, int S, int GMAX, int EPI, int FORM>
+__global__ __launch_bounds__(64 * WM * WN) void gemm_ring_kernel(GemmParams p) {
+    constexpr int NT = 64 * WM * WN, BM = WM * SM * 16, BN = WN * SN * 16;
+    constexpr int kImage = (BM + BN) * 128, kRounds = kImage / 16 / NT;
+    constexpr bool kSilu = EPI == kGemmSilu;
+    static_assert(!kSilu || SN == 2, "the gated FFN pairs gate and up sub-tiles");
+    static_assert(kImage % (16 * NT) == 0, "whole load rounds");
+    static_assert(S == 3 || S == 4, "images of the ring");
+    // one array an image (reads of one are seen not to alias the loads into the others)
+    __shared__ __align__(16) int8_t image0_s[kImage], image1_s[kImage], image2_s[kImage];
+    __shared__ __align__(16) int8_t image3_s[S > 3 ? kImage : 16];
+    auto image = [&](int i) -> int8_t* { return i == 0 ? image0_s : i == 1 ? image1_s : i == 2 ? image2_s : image3_s; };
+    __shared__ __align__(16) float scales_s[BN * GMAX];  // [BN][G]
+
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int wm = wave / WN, wn = wave % WN;
+    const int mtiles = (p.M + BM - 1) / BM;
+    int t = blockIdx.x;
+    if ((gridDim.x & 7) == 0) t = (t & 7) * (gridDim.x >> 3) + (t >> 3);  // one weight panel per XCD
+    const int mt = t % mtiles, nt = t / mtiles;
+    const int m0 = mt * BM, G = p.K / kGroup, chunks = G / 4;
+    auto weight_row = [&](int c) -> int {  // as the chain kernel's
+        if constexpr (kSilu) {
+            const int w = c / 32, j = (c / 16) & 1, o = nt * (BN / 2) + w * 16 + (c & 15);
+            return j == 0 ? o : p.half + o;
+        } else {
+            return nt * BN + c;
+        }
+    };
+    const int r16 = lane & 15, kq = lane >> 4;
+    float sx[SM][4];
+#pragma unroll
+    for (int i = 0; i < SM; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sx[i][r] = p.sx[min(m0 + wm * SM * 16 + i * 16 + 4 * kq + r, p.M - 1)];
+    // 16-byte pieces of the scales: a row's G / 4, in order
+    const int quads = G / 4, slots = BN * quads;
+    for (int q = 0; q < slots; q += NT) {
+        const int sl = q + tid, c = sl / quads, quad = sl - c * quads;
+        if (sl < slots)
+            __builtin_amdgcn_global_load_lds((global_void*)(p.sW + (size_t)min(weight_row(c), p.N - 1) * G + 4 * quad),
+                                             (lds_void*)(scales_s + 4 * (q + 64 * wave)), 16, 0, 0);
+    }
+    const int8_t* src[kRounds];  // this lane's piece of each load round, at column 0
+#pragma unroll
+    for (int q = 0; q < kRounds; ++q) {
+        const int sl = NT * q + tid, row = sl >> 3, piece = (sl & 7) ^ (row & 7);
+        src[q] = (row < BM ? p.X + (size_t)min(m0 + row, p.M - 1) * p.K
+                           : p.W + (size_t)min(weight_row(row - BM), p.N - 1) * p.K) + 16 * piece;
+    }
+    // (written out: of the builtin's loads the compiler keeps a record by array, and
+    // around a loop that record makes every read of an image wait for all of them.
+    // The waits are the counted ones below, and one for all after the loop.)
+    auto request = [&](int ch, int8_t* dst) {
+#pragma unroll
+        for (int q = 0; q < kRounds; ++q) {
+            const uint32_t at = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_void*)dst + 16 * (NT * q + 64 * wave));
+            uint32_t m0;
+            asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off\n\ts_mov_b32 m0, %0"
+                         : "=&s"(m0)
+                         : "s"(at), "v"(src[q] + (size_t)128 * ch)
+                         : "memory");
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < S - 1; ++i) request(min(i, chunks - 1), image(i));
+    // the row scales' wait belongs here (left to their first use, in the loop, it
+    // would wait for every image each time round)
+#pragma unroll
+    for (int i = 0; i < SM; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) asm volatile("" ::"v"(sx[i][r]));
+    float total[SM][SN][4];
+#pragma unroll
+    for (int i = 0; i < SM; ++i)
+#pragma unroll
+        for (int j = 0; j < SN; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) total[i][j][r] = 0.0f;
+    int arow[SM], brow[SN], slot[4];
+    const float* srow[SN];
+#pragma unroll
+    for (int i = 0; i < SM; ++i) arow[i] = (wm * SM * 16 + i * 16 + r16) * 128 + 8 * (kq & 1);
+#pragma unroll
+    for (int j = 0; j < SN; ++j) {
+        brow[j] = (BM + wn * SN * 16 + j * 16 + r16) * 128 + 8 * (kq & 1);
+        srow[j] = scales_s + (wn * SN * 16 + j * 16 + r16) * G;
+    }
+#pragma unroll
+    for (int gg = 0; gg < 4; ++gg) slot[gg] = ((2 * gg + (kq >> 1)) ^ (r16 & 7)) * 16;
+    constexpr int kBias = 0x4b400000;
+    auto chunk = [&](int ch, int i) {  // chunk ch, in image i
+        // the loads of chunk ch (and all before it) are in: S - 2 newer chunks may be outstanding
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm((S - 2) * kRounds));
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        request(min(ch + S - 1, chunks - 1), image((i + S - 1) % S));
+        const int8_t* c = image(i);
+        float4 sv[SN];
+#pragma unroll
+        for (int j = 0; j < SN; ++j) sv[j] = *reinterpret_cast<const float4*>(srow[j] + 4 * ch);
+        long a[4][SM], b[4][SN];
+#pragma unroll
+        for (int gg = 0; gg < 4; ++gg) {
+#pragma unroll
+            for (int k = 0; k < SM; ++k) a[gg][k] = *reinterpret_cast<const long*>(c + arow[k] + slot[gg]);
+#pragma unroll
+            for (int k = 0; k < SN; ++k) b[gg][k] = *reinterpret_cast<const long*>(c + brow[k] + slot[gg]);
+        }
+        // the next group's products are issued before this one's sums are folded
+        v4i acc[2][SM][SN];
+        auto products = [&](int gg) {
+#pragma unroll
+            for (int k = 0; k < SM; ++k)
+#pragma unroll
+                for (int j = 0; j < SN; ++j)
+                    acc[gg & 1][k][j] = __builtin_amdgcn_mfma_i32_16x16x32_i8(a[gg][k], b[gg][j], v4i{kBias, kBias, kBias, kBias}, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        products(0);
+#pragma unroll
+        for (int gg = 0; gg < 4; ++gg) {
+            if (gg < 3) products(gg + 1);
+#pragma unroll
+            for (int k = 0; k < SM; ++k)
+#pragma unroll
+                for (int j = 0; j < SN; ++j) {
+                    const float s = gg == 0 ? sv[j].x : gg == 1 ? sv[j].y : gg == 2 ? sv[j].z : sv[j].w;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const float sum = __int_as_float(acc[gg & 1][k][j][r]) - kSumBias;
+                        if constexpr (FORM == kPanel)
+                            total[k][j][r] = fmaf(sum, s * sx[k][r], total[k][j][r]);  // panel.rs:184-188
+                        else
+                            total[k][j][r] = total[k][j][r] + (sum * s) * sx[k][r];  // neon.rs:180
+                    }
+                }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    for (int ch = 0; ch < chunks; ch += S)
+#pragma unroll
+        for (int i = 0; i < S; ++i)
+            if (ch + i < chunks) chunk(ch + i, i);
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));  // the last requests repeat a chunk nobody reads: in before the block's LDS goes
+
+    // epilogue
+#pragma unroll
+    for (int i = 0; i < SM; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int m = m0 + wm * SM * 16 + i * 16 + 4 * kq + r;
+            if (m >= p.M) continue;
+            if constexpr (kSilu) {
+                const int o = nt * (BN / 2) + wn * 16 + r16;
+                if (o < p.half) p.Y[(size_t)m * p.ldy + o] = silu(total[i][0][r]) * total[i][1][r];
+            } else {
+#pragma unroll
+                for (int j = 0; j < SN; ++j) {
+                    const int n = nt * BN + wn * SN * 16 + j * 16 + r16;
+                    if (n >= p.N) continue;
+                    float* dst = p.Y + (size_t)m * p.ldy + n;
+                    if constexpr (EPI == kGemmResidual)
+                        *dst = *dst + total[i][j][r];
+                    else if constexpr (EPI == kGemmStoreSilu)
+                        *dst = silu(total[i][j][r]);  // stem.rs:76,99: silu after the stage
+                    else
+                        *dst = total[i][j][r];
+                }
+            }
+        }
+}
+
+template <int SM, int SN, int WM, int WN, int S, int GMAX, int EPI, int FORM>
+static void launch_ring(const GemmParams& p, hipStream_t stream) {
+    constexpr int BM = WM * SM * 16, BN = WN * SN * 16;
+    const int mtiles = (p.M + BM - 1) / BM;
+    const int ntiles = EPI == kGemmSilu ? (p.half + BN / 2 - 1) / (BN / 2) : (p.N + BN - 1) / BN;
+    rn_launch((gemm_ring_kernel<SM, SN, WM, WN, S, GMAX, EPI, FORM>), dim3(mtiles * ntiles), dim3(64 * WM * WN), 0, stream, p);
+}
+
 template <int SM, int SN, int WAVES_M, int EPI, int FORM, bool DUMP>
 static void launch_chain(const GemmParams& p, hipStream_t stream) {
     constexpr int BM = WAVES_M * SM * 16, BN = (4 / WAVES_M) * SN * 16;
@@ -701,14 +903,31 @@ static void launch_chain(const GemmParams& p, hipStream_t stream) {
     const int ntiles = EPI == kGemmSilu ? (p.half + BN / 2 - 1) / (BN / 2) : (p.N + BN - 1) / BN;
     const dim3 grid(mtiles * ntiles), block(256);
     if constexpr (!DUMP) {
-        // the whole K panel in LDS for the widths it fits
+        // The whole K panel in LDS for the widths it fits. Rows of 512 from 1024 tiles
+        // of 64 x 64 on go through the ring in those tiles, which read half the bytes
+        // (2048 x 4096 x 512 28.0 us with the quantisation against 30.4, 1000 x 4096
+        // 20.1 against 20.5; the three chunks of 384 columns are too few: 1500 x 3072
+        // 19.1 against 18.3). Wider rows always do: 64 x 64 tiles where there are 512
+        // of them (2048 x 8192 x 2048 155 against 200), else 32-row tiles (1000 x 512 x
+        // 2048 18.4 against 21.3, 1500 x 384 x 1536 17.0 against 18.9).
+        const int n_eff = EPI == kGemmSilu ? 2 * p.half : p.N;
+        const long long tiles64 = (long long)((p.M + 63) / 64) * ((n_eff + 63) / 64);
+        if constexpr (EPI != kGemmRope) {
+            if (p.K == 512 && tiles64 >= 1024) return launch_ring<2, 2, 2, 2, 3, 16, EPI, FORM>(p, stream);
+            if (p.K > 512 && tiles64 >= 512) return launch_ring<2, 2, 2, 2, 3, 64, EPI, FORM>(p, stream);
+            if (p.K > 512) {
+                if constexpr (EPI == kGemmSilu) return launch_ring<1, 2, 2, 2, 3, 64, EPI, FORM>(p, stream);
+                else return launch_ring<1, 1, 2, 2, 4, 64, EPI, FORM>(p, stream);
+            }
+        }
         switch (p.K) {
             case 384: rn_launch((gemm_panel_kernel<384, SM, SN, WAVES_M, EPI, FORM>), grid, block, 0, stream, p); return;
             case 512: rn_launch((gemm_panel_kernel<512, SM, SN, WAVES_M, EPI, FORM>), grid, block, 0, stream, p); return;
-            default: break;
+            default: return;  // launch_gemm takes no other width
         }
+    } else if constexpr (EPI != kGemmRope) {
+        rn_launch((gemm_chain_kernel<SM, SN, WAVES_M, EPI, FORM, DUMP>), grid, block, 0, stream, p);
     }
-    if constexpr (EPI != kGemmRope) rn_launch((gemm_chain_kernel<SM, SN, WAVES_M, EPI, FORM, DUMP>), grid, block, 0, stream, p);
 }
 
 // Tile shape: the one with the most blocks among 64 x 64, 64 x 32, 32 x 64 and

@@ -159,11 +159,13 @@ def test_feed_small_and_ragged_counts(tiny, count):
     (37, 701),     # a ragged last tile behind a cached prefix
     (1600, 645),   # the longest context of the tiles
     (1690, 660),   # the first past it
+    (0, 1000),     # 1024 tiles of 64 x 64 in the gated product where it is 4096 rows wide
 ])
-def test_long_feed_bit_exact(tiny_config, tiny_weights, cached, count):
-    cfg = dict(tiny_config, max_positions=2400)
-    gs = rn.Model(cfg, tiny_weights).session(cached + count)
-    os_ = oracle.OracleModel(cfg, tiny_weights).session(cached + count)
+def test_long_feed_bit_exact(tiny_config, cached, count):
+    cfg = dict(tiny_config, max_positions=2400, ffn=2048)
+    weights = rn.synthetic_weights(cfg, seed=5)
+    gs = rn.Model(cfg, weights).session(cached + count)
+    os_ = oracle.OracleModel(cfg, weights).session(cached + count)
     if cached:
         k, v = rn.synthetic_cache(cfg, cached, "longfeed")
         gs.set_cache(k, v)

@@ -144,6 +144,11 @@ def test_multiply_fused_matches_separate(rows):
     (300, 1000, 512, rn.FORM_PANEL),
     (1500, 384, 1536, rn.FORM_PANEL),
     (600, 1000, 384, rn.FORM_PLANE),
+    # the ring kernel: 1024 or more tiles of 64 x 64 at 512 columns, 512 or more
+    # at wider rows (both forms, ragged tiles), and 32-row tiles at wider rows
+    (1030, 4100, 512, rn.FORM_PANEL),
+    (1500, 1400, 1024, rn.FORM_PLANE),
+    (300, 1000, 2048, rn.FORM_PANEL),
 ])
 def test_multiply_batch_mfma_bit_exact(count, rows, cols, form):
     rng = np.random.default_rng(count * 13 + rows + cols)
