@@ -85,6 +85,22 @@ def test_batch_product_on_the_matrix_cores(bits, group, rows, columns, count):
     assert np.array_equal(acc, acco) and np.array_equal(_bits(y), _bits(yo))
 
 
+# rows of whole 16-byte pieces and rows that are not, narrower than one piece, runs
+# cut by the last column, and counts that leave a block's last wave part empty
+@pytest.mark.parametrize("group,columns,count", [
+    (64, 3, 1), (64, 4, 17), (128, 130, 9), (128, 132, 33), (256, 1000, 5), (256, 1001, 3), (64, 64, 257)])
+def test_prepare_rows_of_any_width(group, columns, count):
+    g, o = _pair(2, group, 2, columns, seed=columns)
+    x = rn.synth_normal(12, "cbp", 1.0, (count, columns))
+    assert np.array_equal(_bits(g.prepare_host(x)), _bits(np.stack([o.prepare(v) for v in x])))
+    # the same rows from an address that is no multiple of 16 bytes
+    xd = rn.DeviceBuffer.from_array(np.concatenate([np.zeros(1, np.float32), x.ravel()]))
+    rd = rn.DeviceBuffer(4 * count * g.padded)
+    g.prepare(xd.ptr + 4, count, rd.ptr)
+    rn.check(rn.lib.rn_stream_synchronize(None))
+    assert np.array_equal(_bits(rd.download(np.float32, (count, g.padded))), _bits(np.stack([o.prepare(v) for v in x])))
+
+
 def test_zero_and_sparse_inputs():
     g, o = _pair(2, 128, 96, 512, seed=1)
     x = np.zeros((2, 512), np.float32)
