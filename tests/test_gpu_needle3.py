@@ -287,6 +287,20 @@ def test_long_feed_equals_pushes(archive):
             assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), layer
 
 
+@pytest.mark.parametrize("heads", [1, 5, 18])
+def test_feed_of_any_attention_width(heads):
+    """The attended rows' codes over half a group, groups the row does not fill, and
+    rows of more than the 1024 values one pass holds."""
+    archive = needle3.synthetic_archive(dict(GEOMETRY, num_heads=heads, num_kv_heads=1))
+    gm, om = needle3.Model(archive), oracle.OracleNeedle3(archive)
+    gs, os_ = gm.session(40), om.session(40)
+    tokens = _tokens(37, seed=heads)
+    gs.feed(tokens)
+    for t in tokens:
+        os_.push(int(t))
+    assert np.array_equal(_bits(gs.logits()), _bits(os_.logits()))
+
+
 @pytest.mark.parametrize("scale", [1e-36, 0.0])
 def test_feed_of_values_of_almost_no_magnitude(archive, scale):
     """Value taps scaled until every value scale is subnormal (weights that a scale
