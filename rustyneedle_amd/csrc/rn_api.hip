@@ -26,6 +26,7 @@
 #include <vector>
 
 #include "../../include/rustyneedle.h"
+#include "rn_flags.hpp"
 #include "rn_internal.hpp"
 #include "rn_matrix.hpp"
 
@@ -192,41 +193,13 @@ int scratch_device(NoAllocDevice** out) {
 }
 }  // namespace
 
-// ---- error flags in pinned host memory ---------------------------------------------
-// A word that a call's kernel writes on an error and the host reads once it has
-// waited for the call's stream: no device allocation, clearing launch or copy back
-// per call (rn_attend_heads with a handful of heads: 42 -> 14 us a call). Words are taken for one call
-// and given back after it, so calls from several threads hold different ones; at
-// most kErrorFlags wait for the next calls, words past that are freed.
 namespace {
-constexpr size_t kErrorFlags = 16;
-std::mutex g_flags_mu;
-std::vector<int32_t*> g_flags;
-
-struct ErrorFlag {
-    int32_t* word = nullptr;
-    ErrorFlag() {
-        {
-            std::lock_guard<std::mutex> lock(g_flags_mu);
-            if (!g_flags.empty()) {
-                word = g_flags.back();
-                g_flags.pop_back();
-            }
-        }
-        if (!word && hipHostMalloc((void**)&word, sizeof(int32_t), hipHostMallocPortable) != hipSuccess) word = nullptr;
-        if (word) *word = 0;
+struct PinnedWords {
+    static int32_t* take() {
+        int32_t* w = nullptr;
+        return hipHostMalloc((void**)&w, sizeof(int32_t), hipHostMallocPortable) == hipSuccess ? w : nullptr;
     }
-    ~ErrorFlag() {
-        if (!word) return;
-        {
-            std::lock_guard<std::mutex> lock(g_flags_mu);
-            if (g_flags.size() < kErrorFlags) {
-                g_flags.push_back(word);
-                return;
-            }
-        }
-        (void)hipHostFree(word);
-    }
+    static void give(int32_t* w) { (void)hipHostFree(w); }
 };
 }  // namespace
 
@@ -777,8 +750,8 @@ int rn_attend_heads(const float* q, const uint16_t* K, const uint16_t* V, const 
     RN_REQUIRE(stride >= 1 && stride <= 16384 && count >= 0, "stride must be 1..16384");
     if (count == 0) return RN_OK;
     hipStream_t s = (hipStream_t)stream;
-    ErrorFlag flag;
-    if (!flag.word) return fail(RN_ERR_MEMORY, "pinned error flag");
+    ErrorFlag<PinnedWords> flag;
+    if (!flag.word()) return fail(RN_ERR_MEMORY, "pinned error flag");
     AttendParams p{};
     p.q = q;
     p.kc = (__half*)K;
@@ -786,11 +759,10 @@ int rn_attend_heads(const float* q, const uint16_t* K, const uint16_t* V, const 
     p.lengths = lengths;
     p.stride = stride;
     p.out = out;
-    p.error = flag.word;
+    p.error = flag.word();
     RN_HIP(launch_attend(p, kAttendRaw, count, 1, stride, s));
     RN_HIP(hipStreamSynchronize(s));
-    const int32_t host_err = *(volatile int32_t*)flag.word;
-    if (host_err) return fail(RN_ERR_ARGUMENT, "a length is outside 1..stride");
+    if (flag.settle()) return fail(RN_ERR_ARGUMENT, "a length is outside 1..stride");
     return RN_OK;
 }
 
