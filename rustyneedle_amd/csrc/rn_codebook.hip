@@ -207,7 +207,7 @@ __global__ __launch_bounds__(1024) void cb_dequantise_kernel(CodebookParams p, i
             if (16 * u + i < p.columns) out[16 * u + i] = v[i];
 }
 
-// The row products of one token (blockIdx.y). A block of
+// The row products of one token (x, y and acc_out are that token's). A block of
 // four waves shares one prologue; each wave owns R = p.rows_per_block rows of a
 // row group of 4R rows, and the block runs p.iters consecutive row groups so
 // that a wide input is quantised once for many rows.
@@ -236,7 +236,6 @@ __device__ __forceinline__ void cb_product_body(const CodebookParams& p, const f
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int R = p.rows_per_block, CPR = p.cpr, G = p.padded / GROUP, runs = p.padded / 16;
     const int BR = NW * R;
-    x += (size_t)blockIdx.y * p.padded;
     uint16_t* nm_s = reinterpret_cast<uint16_t*>(lds);                                 // 12 KB of norms
     int8_t* xq_s = reinterpret_cast<int8_t*>(lds + kNormWindow);                      // [padded]
     int* acc_all = reinterpret_cast<int*>(lds + kNormWindow + p.padded);               // [NW][R][G]
@@ -384,10 +383,9 @@ __device__ __forceinline__ void cb_product_body(const CodebookParams& p, const f
                 else
                     total = total + ((((float)a[g] * norm) * p.lscale) * xs[g]);  // neon.rs:158,180
             }
-            const size_t o = (size_t)blockIdx.y * p.rows + rw + r;
-            y[o] = total;
+            y[rw + r] = total;
             if (acc_out != nullptr)
-                for (int g = 0; g < G; ++g) acc_out[o * G + g] = a[g];
+                for (int g = 0; g < G; ++g) acc_out[(size_t)(rw + r) * G + g] = a[g];
         }
         __syncthreads();  // the norms window and acc_s are read before the next row group replaces them
     };
@@ -404,7 +402,12 @@ __device__ __forceinline__ void cb_product_body(const CodebookParams& p, const f
 template <int BITS, int GROUP, int FORM, int NL>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NL == 8 ? 3 : 1)))
 void cb_product_kernel(CodebookParams p, const float* x, float* y, int32_t* acc_out) {
-    cb_product_body<BITS, GROUP, FORM, NL>(p, x, y, acc_out);
+    // token blockIdx.y; its addresses are formed here, once: an output offset kept
+    // through the body took the 64-column forms two registers past what three waves
+    // a SIMD leave each (12 bytes of scratch a lane)
+    const size_t t = blockIdx.y, G = p.padded / GROUP;
+    cb_product_body<BITS, GROUP, FORM, NL>(p, x + t * p.padded, y + t * p.rows,
+                                           acc_out != nullptr ? acc_out + t * p.rows * G : nullptr);
 }
 
 // Up to four products of one shape in one launch (blockIdx.z picks the job):
