@@ -389,21 +389,26 @@ typedef __attribute__((address_space(3))) void lds_void;
 typedef __attribute__((address_space(1))) void global_void;
 
 // ROWS positions per staged chunk. A context that one 256-row chunk holds is
-// staged once; longer ones take 128-row chunks, half the LDS, so that twice the
-// blocks share a CU: a lone wave a SIMD issues a vector instruction every 5.5
-// cycles, two or more every 2.7 (adds, multiplies) to 4.5 (fp16 products) between
-// them (1000 tokens x 8 heads: 98 us with 256-row chunks, 49 with 128; 256
-// tokens: 9.1 and 9.9).
+// staged once; longer ones can take 128-row chunks, half the LDS, so that twice
+// the blocks share a CU (launch_attend_prefill says when): a lone wave a SIMD
+// issues a vector instruction every 5.5 cycles, two or more every 2.7 (adds,
+// multiplies) to 4.5 (fp16 products) between them (1000 tokens x 8 heads: 98 us
+// with 256-row chunks, 49 with 128; 256 tokens: 9.1 and 9.9).
 template <int QT, int ROWS>
 __global__ __launch_bounds__(256) void attend_prefill_kernel(AttendParams p, int count) {
     constexpr int NT = 256;
     extern __shared__ float scores[];  // [QT][max length]
-    __shared__ __align__(16) __half kv_s[2][ROWS * kHeadDim];  // a chunk of key rows, one of value rows
-    __half *const k_s = kv_s[0], *const v_s = kv_s[1];
+    // (two arrays: in one, a read of the keys would wait for the values under way too)
+    __shared__ __align__(16) __half k_s[ROWS * kHeadDim];  // a chunk of key rows
+    __shared__ __align__(16) __half v_s[ROWS * kHeadDim];  // a chunk of value rows
     __shared__ float q_s[QT][kHeadDim];
     __shared__ float total_s[QT][kClasses];
-    float(*part_s)[kClasses][kHeadDim] = reinterpret_cast<float(*)[kClasses][kHeadDim]>(kv_s);
-    static_assert(QT * kClasses * kHeadDim * 4 <= 2 * ROWS * kHeadDim * 2, "class sums fit in the chunks");
+    // the class sums replace the keys, and the values too where a chunk is small
+    constexpr int kHeld = ROWS * kHeadDim * 2 / (kClasses * kHeadDim * 4);  // queries a buffer holds
+    static_assert(kHeld >= QT || 2 * kHeld == QT, "class sums fit in the chunks");
+    auto part_s = [&](int q) {
+        return reinterpret_cast<float(*)[kHeadDim]>(kHeld >= QT || q < kHeld ? k_s : v_s) + (q % kHeld) * kClasses;
+    };
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     // the last tiles attend the most positions: they go first
@@ -522,11 +527,11 @@ __global__ __launch_bounds__(256) void attend_prefill_kernel(AttendParams p, int
             }
         }
     }
-    __syncthreads();  // the chunks become the class sums
+    if constexpr (kHeld < QT) __syncthreads();  // (the keys' last readers passed a barrier above, the values' not)
 #pragma unroll
     for (int q = 0; q < QT; ++q) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) part_s[q][j][8 * dg + i] = acc[q][i];
+        for (int i = 0; i < 8; ++i) part_s(q)[j][8 * dg + i] = acc[q][i];
         if (dg == 0) total_s[q][j] = total[q];
     }
     __syncthreads();
@@ -536,7 +541,7 @@ __global__ __launch_bounds__(256) void attend_prefill_kernel(AttendParams p, int
             float o = 0.0f, t = 0.0f;
 #pragma unroll
             for (int k = 0; k < kClasses; ++k) {
-                o = o + part_s[q][k][d];
+                o = o + part_s(q)[k][d];
                 t = t + total_s[q][k];
             }
             const float inverse = reciprocal(t);
@@ -761,15 +766,25 @@ hipError_t launch_attend_prefill(const AttendParams& p, int heads, int count, hi
     const int length = p.first + count, pitch = (length + 127) / 128 * 128 + 4;
     const size_t tile_lds = sizeof(float) * kPrefillTileQueries * (size_t)pitch, lds = sizeof(float) * QT * (size_t)length;
     const dim3 grid(heads, (count + QT - 1) / QT);
+    // Half chunks pay only where they let more of the grid run at once: not a grid
+    // that 256-row blocks hold whole (2 to 128 tokens after 1500: 1.16-1.30 ms a prompt
+    // against 1.27-1.40), nor beside scores that leave one block a CU either way
+    // (past 2976 positions: 300 tokens after 3000 4.43 ms against 5.00)
+    auto resident = [&](int rows) {  // blocks the chip's LDS holds
+        const size_t fixed = sizeof(__half) * 2 * rows * kHeadDim + sizeof(float) * QT * (kHeadDim + kClasses);
+        return 256 * (160 * 1024 / (fixed + lds));
+    };
+    const size_t blocks = (size_t)grid.x * grid.y;
+    const bool half_chunks = length > 256 && blocks > resident(256) && resident(128) > resident(256);
     if (count >= 640 && tile_lds <= 148 * 1024)
         rn_launch(attend_prefill_tile_kernel, dim3(heads, (count + kPrefillTileQueries - 1) / kPrefillTileQueries), dim3(1024),
                   tile_lds, stream, p, count, pitch);
     else if (length > kMaxLength)
         return launch_attend(p, kAttendPrefill, heads, count, length, stream);
-    else if (length <= 256)
-        rn_launch((attend_prefill_kernel<QT, 256>), grid, dim3(256), lds, stream, p, count);
-    else
+    else if (half_chunks)
         rn_launch((attend_prefill_kernel<QT, 128>), grid, dim3(256), lds, stream, p, count);
+    else
+        rn_launch((attend_prefill_kernel<QT, 256>), grid, dim3(256), lds, stream, p, count);
     return hipGetLastError();
 }
 

@@ -184,6 +184,34 @@ def test_long_feed_bit_exact(tiny_config, cached, count):
     assert np.array_equal(gv.view(np.uint16), os_.values[:, :, :cached + count])
 
 
+@pytest.mark.parametrize("cached,count", [
+    (1500, 130),   # 264 blocks where 256-row chunks leave one a CU: half chunks
+    (1500, 127),   # 256 blocks: whole chunks
+    (2848, 129),   # 2977 positions leave one block a CU either way: whole chunks
+    (2847, 129),   # two half-chunk blocks still fit
+    (6000, 49),    # too long for whole chunks beside four score rows
+    (6139, 5),     # the longest context of the four-query blocks
+    (6140, 5),     # a block a query past it
+])
+def test_feed_after_a_long_context(tiny_config, cached, count):
+    cfg = dict(tiny_config, layers=1, max_positions=6200)
+    weights = rn.synthetic_weights(cfg, seed=6)
+    gs = rn.Model(cfg, weights).session(cached + count)
+    os_ = oracle.OracleModel(cfg, weights).session(cached + count)
+    k, v = rn.synthetic_cache(cfg, cached, "longcontext")
+    gs.set_cache(k, v)
+    os_.set_cache(k, v)
+    tokens = rn.synth_tokens(rn.SEED, "longcontext.tokens", cfg["vocab"], count)
+    oracle.set_threads(8)
+    try:
+        gs.feed(tokens)
+        os_.feed(tokens)
+        assert np.array_equal(_bits(gs.hidden()), _bits(os_.hidden))
+        assert np.array_equal(_bits(gs.logits()), _bits(os_.logits()))
+    finally:
+        oracle.set_threads(1)
+
+
 def test_clone_is_independent(tiny, tiny_config):
     gm, _ = tiny
     k, v = rn.synthetic_cache(tiny_config, 10, "clone")
