@@ -661,22 +661,33 @@ inline int product_loads(const CodebookParams& p) { return p.cpr < 64 ? 8 : 16; 
 inline int product_rows(const CodebookParams& p) { return min(64, 64 * product_loads(p) / p.cpr); }
 constexpr size_t kProductMaxLds = 64 * 1024;
 
+// The row kernel's plan: rows a wave, consecutive row groups a block (at least 4,
+// or padded / 1024 for a wide input, whose prologue then serves them all, while
+// the grid keeps at least 512 blocks; each group's loads are in flight during the
+// previous group's decode), blocks a token
+struct RowsPlan {
+    int rows, iters, blocks;
+};
+inline RowsPlan plan_rows(const CodebookParams& p) {
+    RowsPlan r;
+    r.rows = product_rows(p);
+    const int groups = (p.rows + 4 * r.rows - 1) / (4 * r.rows);
+    r.iters = max(1, min(max(4, p.padded / 1024), groups / 512));
+    r.blocks = (groups + r.iters - 1) / r.iters;
+    return r;
+}
+
 template <int BITS, int GROUP, int FORM>
 hipError_t launch_product_rows(const CodebookParams& p, const float* x, int count, float* y, int32_t* acc,
                             hipStream_t stream) {
-    const int nl = product_loads(p);
+    const RowsPlan plan = plan_rows(p);
     CodebookParams q = p;
-    q.rows_per_block = product_rows(p);
-    const size_t lds = product_lds(p, q.rows_per_block);
+    q.rows_per_block = plan.rows;
+    q.iters = plan.iters;
+    const size_t lds = product_lds(p, plan.rows);
     if (lds > kProductMaxLds) return hipErrorInvalidValue;
-    // consecutive row groups per block (at least 4, or padded / 1024 for a wide
-    // input, whose prologue then serves them all), while the grid keeps at
-    // least 512 blocks; each group's loads are in flight during the previous
-    // group's decode
-    const int groups = (p.rows + 4 * q.rows_per_block - 1) / (4 * q.rows_per_block);
-    q.iters = max(1, min(max(4, p.padded / 1024), groups / 512));
-    const dim3 grid((groups + q.iters - 1) / q.iters, count);
-    if (nl == 8)
+    const dim3 grid(plan.blocks, count);
+    if (product_loads(p) == 8)
         rn_launch(cb_product_kernel<BITS, GROUP, FORM, 8>, grid, dim3(256), lds, stream, q, x, y, acc);
     else
         rn_launch(cb_product_kernel<BITS, GROUP, FORM, 16>, grid, dim3(256), lds, stream, q, x, y, acc);
@@ -711,19 +722,26 @@ hipError_t launch_tile(const CodebookParams& p, const float* x, int count, float
 template <int BITS, int GROUP, int FORM>
 hipError_t launch_product_g(const CodebookParams& p, const float* x, int count, float* y, int32_t* acc,
                             hipStream_t stream) {
-    // One token a block while the whole batch is small: the blocks then outnumber
-    // the tile kernel's and each quantises one row (5.4 against 5.8 us at 16
-    // tokens x 2000 rows x 1024 columns of 2 bits, 6.4 against 5.1 us at 64 x
-    // 2000 x 384; 9.7 against 8.6 at 16 x 2000 x 2560). Rows too wide for a tile's
-    // LDS stay there too.
-    const long long weights = (long long)count * p.rows * p.padded;
+    // One token a block (the row kernel) while its blocks fit the chip in two rounds
+    // or so; past that the tile kernel, whose cost is its blocks' quantisation, a chain
+    // over the columns, until there is work for all of its waves. Blocks, columns and
+    // tokens decide, not the bytes: 2-bit 256 tokens x 2048 x 64 are 2048 blocks (9.7
+    // us, tiles 4.8); 4-bit 64 x 200 x 4096 are 448 (10.7 us, tiles 15.5); 2-bit 2 x 8192
+    // x 3000 are 410 (6.7 us, tiles 8.8). Narrow rows (under 18 pieces of 16 bytes, whose
+    // tiles are cheap) stay on it up to 2^25 (token, weight) pairs only, and so do many tokens
+    // by few rows (512 x 48 x 2048 at 4 bits: tiles 8.0 us against 9.9). Rows too
+    // wide for a tile's LDS always do.
+    const long long weights = (long long)count * p.rows * p.padded, blocks = (long long)count * plan_rows(p).blocks;
     const bool fits = p.padded / p.group <= 32 * kTileNormLoads && tile_lds(p, 16) <= kTileMaxLds;
-    if (count == 1 || !fits || (weights <= (1ll << 25) && count <= 65535))
+    const bool wide_rows = p.cpr >= 18 && count <= 256 && blocks <= (p.cpr >= 128 ? 768 : 512);
+    if (count == 1 || !fits || wide_rows || (weights <= (1ll << 25) && blocks <= 768))
         return launch_product_rows<BITS, GROUP, FORM>(p, x, count, y, acc, stream);
     if (acc != nullptr) return launch_tile<BITS, GROUP, FORM, 1, true>(p, x, count, y, acc, stream);
     // two 16-token sub-tiles a wave halve the decode per product and double the
     // block's quantisation: they pay once a block has some hundred rows (4-bit
-    // indices cost three times the 2-bit decode)
+    // indices cost three times the 2-bit decode). Over 48 to 65536 rows of 64 to 4096
+    // columns: at 4 bits 0.75-0.98 of the speed between 2^19 and 2^19.5 (token, row)
+    // pairs, 1.01-1.13 from 2^20; at 2 bits 0.95-1.16 at 2^20.5, 1.08-1.23 at 2^21.5
     const bool wide = count > 16 && (long long)p.rows * count > (p.bits == 4 ? 1ll << 20 : 3ll << 20) &&
                       tile_lds(p, 32) <= kTileMaxLds;
     return wide ? launch_tile<BITS, GROUP, FORM, 2>(p, x, count, y, acc, stream)
@@ -860,17 +878,15 @@ namespace {
 template <int BITS, int GROUP, int FORM>
 hipError_t launch_jobs_t(CodebookJobs jobs, int n, hipStream_t stream) {
     const CodebookParams& p = jobs.job[0].p;
-    const int nl = product_loads(p), R = product_rows(p);
-    const size_t lds = product_lds(p, R);
+    const RowsPlan plan = plan_rows(p);
+    const size_t lds = product_lds(p, plan.rows);
     if (lds > kProductMaxLds) return hipErrorInvalidValue;
-    const int groups = (p.rows + 4 * R - 1) / (4 * R);
-    const int iters = max(1, min(max(4, p.padded / 1024), groups / 512));
     for (int i = 0; i < n; ++i) {
-        jobs.job[i].p.rows_per_block = R;
-        jobs.job[i].p.iters = iters;
+        jobs.job[i].p.rows_per_block = plan.rows;
+        jobs.job[i].p.iters = plan.iters;
     }
-    const dim3 grid((groups + iters - 1) / iters, 1, n);
-    if (nl == 8)
+    const dim3 grid(plan.blocks, 1, n);
+    if (product_loads(p) == 8)
         rn_launch(cb_product_jobs_kernel<BITS, GROUP, FORM, 8>, grid, dim3(256), lds, stream, jobs);
     else
         rn_launch(cb_product_jobs_kernel<BITS, GROUP, FORM, 16>, grid, dim3(256), lds, stream, jobs);

@@ -74,6 +74,27 @@ def test_batch_product(bits, group, rows, columns, count):
     (4, 128, 9001, 130, 130),    # 32-token tiles of 4-bit indices
 ])
 def test_batch_product_on_the_matrix_cores(bits, group, rows, columns, count):
+    _batch_equals_oracle(bits, group, rows, columns, count)
+
+
+# both sides of the lines between the row kernel and the tiles: its blocks, the
+# pieces of a row, the tokens
+@pytest.mark.parametrize("bits,group,rows,columns,count", [
+    (4, 128, 200, 4096, 109),    # 128 pieces a row, 763 blocks: rows
+    (4, 128, 200, 4096, 110),    # 770: tiles
+    (2, 64, 517, 1100, 102),     # 18 pieces, 510 blocks: rows
+    (2, 64, 517, 1100, 103),     # 515: tiles
+    (2, 64, 517, 1024, 102),     # 16 pieces: tiles
+    (5, 64, 2048, 64, 96),       # one piece, 768 blocks: rows
+    (5, 64, 2048, 64, 97),       # 776: tiles
+    (4, 256, 40, 3000, 256),     # 256 blocks of 256 tokens: rows
+    (4, 256, 48, 3000, 257),     # 257 tokens: tiles
+])
+def test_batch_product_by_rows_or_tiles(bits, group, rows, columns, count):
+    _batch_equals_oracle(bits, group, rows, columns, count)
+
+
+def _batch_equals_oracle(bits, group, rows, columns, count):
     g, o = _pair(bits, group, rows, columns, seed=count)
     x = rn.synth_normal(9, "cbt", 1.0, (count, columns))
     x[count - 1] *= 1e3
