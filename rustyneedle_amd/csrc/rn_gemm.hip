@@ -283,8 +283,8 @@ __global__ __launch_bounds__(1024) void gemm_split_kernel(GemmParams p) {
 }
 
 // ---- the chain GEMM: group chains kept in the MFMA result registers ----------
-// (the form that also writes the int32 sums out; products without them take the
-// panel and ring forms below)
+// (the form that also writes the int32 sums out; products without them take it at
+// one band of sizes, launch_wide, and otherwise the panel and ring forms below)
 //
 // A 256-thread block (4 waves, WAVES_M x (4 / WAVES_M)) owns a BM x BN output
 // tile; each wave owns SM x SN sub-tiles of 16 x 16, and each lane 4 outputs per
@@ -896,8 +896,36 @@ static void launch_ring(const GemmParams& p, hipStream_t stream) {
     rn_launch((gemm_ring_kernel<SM, SN, WM, WN, S, GMAX, EPI, FORM>), dim3(mtiles * ntiles), dim3(64 * WM * WN), 0, stream, p);
 }
 
+// Rows wider than 512: tiles of 32 x 32, 64 x 32 or 64 x 64 through the ring, by how
+// their blocks divide over 256 CUs. A 64 x 64 block takes a CU some 20 us at 2048
+// columns alone or with a second one beside it, so an odd number a CU wastes half a
+// round: 64 x 32 blocks then (2048 columns, 700 x 3072, 528 tiles of 64 x 64: 31.7 us,
+// 64 x 64 40.5; 600 x 4096, 640 tiles: 32.2 and 39.6; 512 tiles 28.9 and 24.3).
+// Under 512 such tiles 32 x 32 blocks (128 x 2048: 12.3 us, 64 x 32 15.2), but at 2048
+// columns from the fourth a CU on 64 x 32 (400 x 2048: 16.5 us against 19.9), and while
+// that would put a third one on a few CUs, five 32 x 32 a CU, the chain kernel, whose
+// blocks need less LDS (600 x 2048: 22.4 us, 64 x 32 23.4, 32 x 32 23.9). Both forms
+// within 4% of these.
+template <int EPI, int FORM>
+static void launch_wide(const GemmParams& p, hipStream_t stream) {
+    auto tiles = [&](int bm, int bn) { return ((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn); };
+    const int large = tiles(64, 64), small_per_cu = (tiles(32, 32) + 255) / 256, large_per_cu = (large + 255) / 256;
+    if (large >= 512) {
+        if (large_per_cu == 3 || large_per_cu == 5) return launch_ring<2, 1, 2, 2, 3, 64, EPI, FORM>(p, stream);
+        return launch_ring<2, 2, 2, 2, 3, 64, EPI, FORM>(p, stream);
+    }
+    if constexpr (EPI != kGemmStoreSilu) {  // (1152 and 1536 columns)
+        if (p.K == 2048 && small_per_cu >= 4 && small_per_cu <= 6) {
+            if (small_per_cu != 5) return launch_ring<2, 1, 2, 2, 3, 64, EPI, FORM>(p, stream);
+            rn_launch((gemm_chain_kernel<1, 1, 2, EPI, FORM, false>), dim3(tiles(32, 32)), dim3(256), 0, stream, p);
+            return;
+        }
+    }
+    launch_ring<1, 1, 2, 2, 4, 64, EPI, FORM>(p, stream);
+}
+
 template <int SM, int SN, int WAVES_M, int EPI, int FORM, bool DUMP>
-static void launch_chain(const GemmParams& p, hipStream_t stream) {
+static hipError_t launch_chain(const GemmParams& p, hipStream_t stream) {
     constexpr int BM = WAVES_M * SM * 16, BN = (4 / WAVES_M) * SN * 16;
     const int mtiles = (p.M + BM - 1) / BM;
     const int ntiles = EPI == kGemmSilu ? (p.half + BN / 2 - 1) / (BN / 2) : (p.N + BN - 1) / BN;
@@ -907,27 +935,28 @@ static void launch_chain(const GemmParams& p, hipStream_t stream) {
         // of 64 x 64 on go through the ring in those tiles, which read half the bytes
         // (2048 x 4096 x 512 28.0 us with the quantisation against 30.4, 1000 x 4096
         // 20.1 against 20.5; the three chunks of 384 columns are too few: 1500 x 3072
-        // 19.1 against 18.3). Wider rows always do: 64 x 64 tiles where there are 512
-        // of them (2048 x 8192 x 2048 155 against 200), else 32-row tiles (1000 x 512 x
-        // 2048 18.4 against 21.3, 1500 x 384 x 1536 17.0 against 18.9).
-        const int n_eff = EPI == kGemmSilu ? 2 * p.half : p.N;
-        const long long tiles64 = (long long)((p.M + 63) / 64) * ((n_eff + 63) / 64);
+        // 19.1 against 18.3). Wider rows always do.
         if constexpr (EPI != kGemmRope) {
-            if (p.K == 512 && tiles64 >= 1024) return launch_ring<2, 2, 2, 2, 3, 16, EPI, FORM>(p, stream);
-            if (p.K > 512 && tiles64 >= 512) return launch_ring<2, 2, 2, 2, 3, 64, EPI, FORM>(p, stream);
-            if (p.K > 512) {
-                if constexpr (EPI == kGemmSilu) return launch_ring<1, 2, 2, 2, 3, 64, EPI, FORM>(p, stream);
-                else return launch_ring<1, 1, 2, 2, 4, 64, EPI, FORM>(p, stream);
+            const int n_eff = EPI == kGemmSilu ? 2 * p.half : p.N;
+            if (p.K == 512 && (long long)((p.M + 63) / 64) * ((n_eff + 63) / 64) >= 1024) {
+                launch_ring<2, 2, 2, 2, 3, 16, EPI, FORM>(p, stream);
+                return hipGetLastError();
             }
+            if constexpr (EPI != kGemmSilu)
+                if (p.K > 512) {
+                    launch_wide<EPI, FORM>(p, stream);
+                    return hipGetLastError();
+                }
         }
         switch (p.K) {
-            case 384: rn_launch((gemm_panel_kernel<384, SM, SN, WAVES_M, EPI, FORM>), grid, block, 0, stream, p); return;
-            case 512: rn_launch((gemm_panel_kernel<512, SM, SN, WAVES_M, EPI, FORM>), grid, block, 0, stream, p); return;
-            default: return;  // launch_gemm takes no other width
+            case 384: rn_launch((gemm_panel_kernel<384, SM, SN, WAVES_M, EPI, FORM>), grid, block, 0, stream, p); break;
+            case 512: rn_launch((gemm_panel_kernel<512, SM, SN, WAVES_M, EPI, FORM>), grid, block, 0, stream, p); break;
+            default: return hipErrorInvalidValue;  // a gated product or rotary rows of another width
         }
-    } else if constexpr (EPI != kGemmRope) {
+    } else {
         rn_launch((gemm_chain_kernel<SM, SN, WAVES_M, EPI, FORM, DUMP>), grid, block, 0, stream, p);
     }
+    return hipGetLastError();
 }
 
 // Tile shape: the one with the most blocks among 64 x 64, 64 x 32, 32 x 64 and
@@ -955,14 +984,14 @@ static int chain_pick(const GemmParams& p) {
 }
 
 template <int EPI, int FORM, bool DUMP>
-static void launch_chain_shape(const GemmParams& p, int pick, hipStream_t stream) {
+static hipError_t launch_chain_shape(const GemmParams& p, int pick, hipStream_t stream) {
     switch (pick) {
-        case 0: launch_chain<2, 2, 2, EPI, FORM, DUMP>(p, stream); break;
-        case 1: launch_chain<1, 2, 4, EPI, FORM, DUMP>(p, stream); break;
-        case 2: launch_chain<1, 2, 2, EPI, FORM, DUMP>(p, stream); break;
+        case 0: return launch_chain<2, 2, 2, EPI, FORM, DUMP>(p, stream);
+        case 1: return launch_chain<1, 2, 4, EPI, FORM, DUMP>(p, stream);
+        case 2: return launch_chain<1, 2, 2, EPI, FORM, DUMP>(p, stream);
         default:
-            if constexpr (EPI != kGemmSilu) launch_chain<1, 1, 2, EPI, FORM, DUMP>(p, stream);
-            break;
+            if constexpr (EPI != kGemmSilu) return launch_chain<1, 1, 2, EPI, FORM, DUMP>(p, stream);
+            return hipErrorInvalidValue;
     }
 }
 
@@ -1018,8 +1047,7 @@ static hipError_t launch_product(const GemmParams& p, hipStream_t stream) {
                                                       const_cast<float*>(p.sx), nullptr, stream);
             if (e != hipSuccess) return e;
         }
-        launch_chain<1, 1, 2, kGemmRope, FORM, false>(p, stream);
-        return hipGetLastError();
+        return launch_chain<1, 1, 2, kGemmRope, FORM, false>(p, stream);
     } else {
     const int pick = p.K == 1152 ? (EPI == kGemmSilu ? 2 : 3) : chain_pick<EPI>(p);
     const int n_eff = EPI == kGemmSilu ? 2 * p.half : p.N;
@@ -1034,8 +1062,8 @@ static hipError_t launch_product(const GemmParams& p, hipStream_t stream) {
         if (e != hipSuccess) return e;
     }
     if (pick >= 0)
-        launch_chain_shape<EPI, FORM, DUMP>(p, pick, stream);
-    else if (fused)
+        return launch_chain_shape<EPI, FORM, DUMP>(p, pick, stream);
+    if (fused)
         launch_by_rows<EPI, FORM, DUMP, kRowsQuant>(p, stream);
     else if (fused_norm && reread <= ((size_t)8 << 20))
         launch_split<16, 16, 32, EPI, FORM, DUMP, kRowsNormQuant>(p, stream);

@@ -149,6 +149,13 @@ def test_multiply_fused_matches_separate(rows):
     (1030, 4100, 512, rn.FORM_PANEL),
     (1500, 1400, 1024, rn.FORM_PLANE),
     (300, 1000, 2048, rn.FORM_PANEL),
+    # wide rows by the blocks a CU takes: 64 x 32 tiles (528 of 64 x 64, and 800 of
+    # 32 x 32 at 2048 columns, ragged), the chain kernel (1045 of 32 x 32 there)
+    (700, 3071, 1024, rn.FORM_PANEL),
+    (395, 1961, 2048, rn.FORM_PLANE),
+    (395, 1961, 2048, rn.FORM_PANEL),
+    (600, 1745, 2048, rn.FORM_PANEL),
+    (600, 1745, 2048, rn.FORM_PLANE),
 ])
 def test_multiply_batch_mfma_bit_exact(count, rows, cols, form):
     rng = np.random.default_rng(count * 13 + rows + cols)
