@@ -344,13 +344,15 @@ hipError_t launch_attend(const AttendParams& p, int mode, int grid_x, int grid_y
             // one sequence: its loads go out before its position is read. Many ragged
             // ones clamp their loads to their own positions: while the blocks do not
             // fill the chip, passes of 384 keys and 288 values (20 sequences of up to
-            // 700: 718 us a step against 740 with 640 and 576); once they do, short
+            // 700: 736 us a step against 764 with 640 and 576; up to 256: 625 against
+            // 651), but a single pass where only the larger one holds the cache (20 of up to
+            // 420: 677 against 691; equal at 576, ahead again from 600). Once they do, short
             // caches take 256-thread blocks, four a CU (96 sequences of up to 60: 691
             // against 792), long ones a single pass up to 576 positions (64 of up to
             // 512: 782 us a step, 812 in 256-position passes).
             if (grid_y == 1)
                 rn_launch((attend_kernel<kAttendDecode, 6, 12, false>), grid, dim3(256), lds, stream, p);
-            else if (grid_x * grid_y < 256)
+            else if (grid_x * grid_y < 256 && !(max_length > 384 && max_length <= 576))
                 rn_launch((attend_kernel<kAttendDecode, 3, 9, true, 512>), grid, dim3(512), lds, stream, p);
             else if (max_length <= 256)
                 rn_launch((attend_kernel<kAttendDecode, 4, 8, true>), grid, dim3(256), lds, stream, p);
@@ -364,7 +366,10 @@ hipError_t launch_attend(const AttendParams& p, int mode, int grid_x, int grid_y
             // the length first: a ragged problem's blocks fetch its own rows only, in
             // short passes whose registers leave four blocks a CU (512 heads of up to 512
             // positions 20.1 us a call against 25.3 with the rows requested before the
-            // length); a few long ones take 512 threads (4 x 4000: 27.1 against 30.6)
+            // length). Few long ones take 512 threads: from 769 positions, three passes of
+            // 256 (a call of 32 heads: 768 positions 20.1 us against 19.7, 900 20.3 against
+            // 21.2, 4000 37.9 against 48.9); not measured past 64 heads when it was set,
+            // 512 threads also lead at 65 to 200 (128 x 2000 29.5 against 33.1)
             if (grid_x <= 64 && p.stride > 768)
                 rn_launch((attend_kernel<kAttendRaw, 5, 18, true, 512>), grid, dim3(512), lds, stream, p);
             else

@@ -289,6 +289,35 @@ def test_batch_decode_with_a_full_chip(tiny, tiny_config, heads_blocks, capacity
         assert np.array_equal(_bits(b.logits()[i]), _bits(s.logits())), i
 
 
+@pytest.mark.parametrize("count,capacity,lengths", [
+    (9, 384, [285, 286, 287, 288, 289, 380]),        # under 256 blocks, one pass of keys, two of values
+    (9, 390, [287, 289, 382, 383, 384, 386]),        # one pass of the larger instance
+    (9, 576, [382, 385, 570, 572]),
+    (9, 960, [285, 383, 384, 385, 575, 576, 577, 650, 767, 768, 769, 865, 956]),  # and several of the smaller
+    (33, 960, [574, 575, 576, 577, 638, 639, 640, 641, 956]),                    # over 256: several of the larger
+])
+def test_batch_decode_passes(tiny_config, count, capacity, lengths):
+    """Lengths around the passes of every attention instance, beside short sequences."""
+    cfg = dict(tiny_config, layers=1, max_positions=1024)
+    gm = rn.Model(cfg, rn.synthetic_weights(cfg, seed=9))
+    steps = 4
+    lengths = [1, 31, 200] + lengths
+    count = max(count, len(lengths))
+    lengths = np.array([lengths[i % len(lengths)] for i in range(count)])
+    assert lengths.max() + steps <= capacity
+    first = rn.synth_tokens(rn.SEED, "passes.first", cfg["vocab"], count)
+    k, v = rn.synthetic_cache(cfg, capacity, "passes")
+    b = rn.Batch(gm, count, capacity)
+    for i, n in enumerate(lengths):
+        b.set_cache(i, np.ascontiguousarray(k[:, :, :n]), np.ascontiguousarray(v[:, :, :n]))
+    ids = b.decode_greedy(first, steps)
+    for i in range(min(count, 16)):
+        s = gm.session(capacity)
+        s.set_cache(np.ascontiguousarray(k[:, :, :lengths[i]]), np.ascontiguousarray(v[:, :, :lengths[i]]))
+        assert ids[i].tolist() == s.decode_greedy(int(first[i]), steps).tolist(), (i, lengths[i])
+        assert np.array_equal(_bits(b.logits()[i]), _bits(s.logits())), (i, lengths[i])
+
+
 def test_full_decode_workload_bit_identical():
     """The batch-1 decode workload at full size: 20 layers, d 512, vocab 8192,
     fp16 cache pre-filled to 256, 64 greedy tokens — ids equal the oracle's."""
