@@ -566,7 +566,8 @@ constexpr int kPrefillTileQueries = 16;
 // v_mfma_f32_16x16x1_4b adds one product to +0, which rounds it exactly as the
 // vector multiply does (equal on all inputs tried, subnormal, infinite and NaN
 // ones included, but for the sign of a zero, which no later addition sees: the
-// running sums start at +0 and are never -0), and the vector unit only adds.
+// running sums start at +0 and are never -0; test_long_feed_of_extreme_scores_and_values
+// keeps it so for products and sums that are subnormal), and the vector unit only adds.
 // It forms 28 products a cycle, the vector unit 14 of a fp16 operand; the two do
 // not overlap. Its four blocks are four independent outer products of 16 queries:
 //   1. scores: block b takes sub-sum 4 m + b of the T2 tree, in step (m, i) its

@@ -157,8 +157,10 @@ def test_feed_small_and_ragged_counts(tiny, count):
     (0, 300),      # past the 256 rows one staged chunk holds
     (0, 640),      # whole 16-query tiles on the matrix instructions
     (37, 701),     # a ragged last tile behind a cached prefix
-    (1600, 645),   # the longest context of the tiles
-    (1690, 660),   # the first past it
+    (1600, 645),   # 2245 positions, on the tiles
+    (1690, 660),   # 2350, past them
+    (1664, 640),   # the longest context of the tiles, 2304 positions
+    (1665, 640),   # the first past it
     (0, 1000),     # 1024 tiles of 64 x 64 in the gated product where it is 4096 rows wide
 ])
 def test_long_feed_bit_exact(tiny_config, cached, count):
@@ -210,6 +212,54 @@ def test_feed_after_a_long_context(tiny_config, cached, count):
         assert np.array_equal(_bits(gs.logits()), _bits(os_.logits()))
     finally:
         oracle.set_threads(1)
+
+
+@pytest.mark.parametrize("tiny_sums", [False, True])
+def test_long_feed_of_extreme_scores_and_values(tiny_config, tiny_sums):
+    """640 tokens and more, whose products the f32 matrix instructions form, over
+    cached keys that spread the scores far past the exponent's floor and values of
+    zeros of both signs, subnormals and tiny magnitudes. With `tiny_sums` every
+    position of weight holds zeros and the rest subnormals, so that each product of a
+    weight at the floor (2^-126 and a little) and each sum is subnormal; the output
+    matrix's scales bring them back beside the residual stream."""
+    cached, count = 300, 704
+    cfg = dict(tiny_config, layers=2, max_positions=1024)
+    weights = rn.synthetic_weights(cfg, seed=8)
+    rng = np.random.default_rng(8)
+    k, v = rn.synthetic_cache(cfg, cached, "extreme")
+    shape = (cfg["layers"], cfg["heads"])
+    # pairs of opposite keys far along one dimension: one of them scores high with any query
+    for i in range(16):
+        far = np.zeros((*shape, 64), np.float16)
+        np.put_along_axis(far, rng.integers(0, 64, (*shape, 1)), np.float16(3000.0), -1)
+        k[:, :, 2 * i], k[:, :, 2 * i + 1] = far, -far
+    if tiny_sums:
+        v[:] = (rng.uniform(-6e-5, 6e-5, v.shape)).astype(np.float16)  # subnormal in 16 bits
+        v[:, :, :32] = np.where(rng.integers(0, 2, v[:, :, :32].shape), np.float16(0.0), np.float16(-0.0))
+        for layer in weights["layers"]:
+            layer["qkv"][1][2 * cfg["d_model"]:] *= np.float32(1e-9)  # the fed tokens' own values: zeros and subnormals
+            layer["out"][1][:] *= np.float32(1e39 / 2 ** 7)
+    else:
+        k[:, :, 32::3] *= np.float16(30.0)
+        v[:, :, 0::4] = (rng.uniform(-1, 1, v[:, :, 0::4].shape) * 1e-7).astype(np.float16)
+        v[:, :, 1::4] = np.where(rng.integers(0, 2, v[:, :, 1::4].shape), np.float16(0.0), np.float16(-0.0))
+        v[:, :, 2::4] *= np.float16(6e4 / 8)
+    gs = rn.Model(cfg, weights).session(cached + count)
+    os_ = oracle.OracleModel(cfg, weights).session(cached + count)
+    gs.set_cache(k, v)
+    os_.set_cache(k, v)
+    tokens = rn.synth_tokens(rn.SEED, "extreme.tokens", cfg["vocab"], count)
+    oracle.set_threads(8)
+    try:
+        gs.feed(tokens)
+        os_.feed(tokens)
+    finally:
+        oracle.set_threads(1)
+    assert np.all(np.isfinite(os_.hidden))
+    assert np.array_equal(_bits(gs.hidden()), _bits(os_.hidden))
+    gk, gv = gs.get_cache()
+    assert np.array_equal(gk.view(np.uint16), os_.keys[:, :, :cached + count])
+    assert np.array_equal(gv.view(np.uint16), os_.values[:, :, :cached + count])
 
 
 def test_clone_is_independent(tiny, tiny_config):
