@@ -71,9 +71,10 @@ __device__ __forceinline__ float score_row(const float* q16, const uint4& ka, co
 
 // KC key passes of NT/4 rows and VC value positions per thread are issued
 // together (NT/4*KC and 32*VC positions); NT threads, 4 lanes per key row and
-// NT/32 lanes per position class. POS_FIRST (decode of many sequences): read
-// the position before the cache loads and clamp them to it, instead of to the
-// capacity, so that short caches do not fetch the rows of long ones. Passes and
+// NT/32 lanes per position class. POS_FIRST (decode of many sequences, and the
+// raw form): read the position (the length) before the cache loads and clamp them
+// to it, instead of to the capacity, so that short caches do not fetch the rows of
+// long ones. Passes and
 // value slots past the length are skipped per wave (they add nothing).
 template <int MODE, int KC, int VC, bool POS_FIRST, int NT = 256>
 // (512-thread blocks are held to 128 VGPRs, so that two blocks share a CU)
@@ -121,7 +122,6 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT >= 512 ? 
         K = p.kc + (size_t)i * p.stride * kHeadDim;
         V = p.vc + (size_t)i * p.stride * kHeadDim;
         out = p.out + (size_t)i * kHeadDim;
-        rows = p.stride;
     }
 
     // the new q/k/v row and its rotary factors (decoding many sequences): requested
@@ -138,10 +138,11 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT >= 512 ? 
             nv[1] = row[2 * p.d_model + kHeadDim / 2];
         }
     }
-    if constexpr (MODE == kAttendRaw && POS_FIRST) {
+    if constexpr (MODE == kAttendRaw) {
+        static_assert(POS_FIRST, "the raw form reads its length first");
         rows = p.lengths[blockIdx.x];
         if (rows < 1 || rows > p.stride) {
-            if (tid == 0) *p.error = 4;
+            if (tid == 0) *p.error = 4;  // (host memory: stores of one value, no atomic)
             return;
         }
     } else if constexpr (POS_FIRST) {
@@ -221,12 +222,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT >= 512 ? 
         has_new = false;
         if (tid < kHeadDim) q_s[tid] = p.q[(size_t)blockIdx.y * p.d_model + blockIdx.x * kHeadDim + tid];
     } else {
-        nglobal = POS_FIRST ? rows : p.lengths[blockIdx.x];
+        nglobal = rows;
         has_new = false;
-        if (nglobal < 1 || nglobal > p.stride) {
-            if (tid == 0) *p.error = 4;  // (host memory: stores of one value, no atomic)
-            return;
-        }
         if (tid < kHeadDim) q_s[tid] = p.q[(size_t)blockIdx.x * kHeadDim + tid];
     }
     const int length = nglobal + (has_new ? 1 : 0);

@@ -295,9 +295,7 @@ __global__ __launch_bounds__(1024) void gemm_split_kernel(GemmParams p) {
 // leaves the registers. K streams through LDS in chunks of 4 groups (128 bytes
 // of every tile row), double-buffered: the next chunk's operand pieces and
 // weight scales are requested before the current chunk's MFMAs, and written to
-// the other buffer after them; one barrier per chunk. For the gated FFN
-// (SN = 2) sub-tile column 0 holds gate rows and column 1 the matching up rows,
-// so silu(gate) * up needs no exchange.
+// the other buffer after them; one barrier per chunk.
 constexpr int kChunkGroups = 4;                  // groups per K chunk
 constexpr int kChunkBytes = kChunkGroups * kGroup;  // 128
 constexpr int kChunkPitch = kChunkBytes + 16;    // LDS row pitch: 16-byte aligned, rows start on different banks
@@ -306,8 +304,7 @@ template <int SM, int SN, int WAVES_M, int EPI, int FORM, bool DUMP>
 __global__ __launch_bounds__(256) void gemm_chain_kernel(GemmParams p) {
     constexpr int WAVES_N = 4 / WAVES_M;
     constexpr int BM = WAVES_M * SM * 16, BN = WAVES_N * SN * 16;
-    constexpr bool kSilu = EPI == kGemmSilu;
-    static_assert(!kSilu || SN == 2, "the gated FFN pairs gate and up sub-tiles");
+    static_assert(EPI == kGemmStore || EPI == kGemmResidual, "plain and residual products");
     constexpr int kPieces = (BM + BN) * (kChunkBytes / 16);  // 16-byte pieces per chunk
     constexpr int kPer = (kPieces + 255) / 256;
     __shared__ __align__(16) int8_t a_s[2][BM][kChunkPitch];
@@ -322,21 +319,6 @@ __global__ __launch_bounds__(256) void gemm_chain_kernel(GemmParams p) {
     const int m0 = mt * BM;
     const int G = p.K / kGroup, chunks = G / kChunkGroups;
 
-    // weight row of local tile column c (silu: wave column block wn holds 16
-    // outputs; its sub-tile column 0 is their gate rows, column 1 their up rows)
-    auto weight_row = [&](int c) -> int {
-        if constexpr (kSilu) {
-            const int w = c / 32, j = (c / 16) & 1, o = nt * (BN / 2) + w * 16 + (c & 15);
-            return j == 0 ? o : p.half + o;
-        } else {
-            return nt * BN + c;
-        }
-    };
-    auto row_ok = [&](int c) -> bool {
-        if constexpr (kSilu) return nt * (BN / 2) + (c / 32) * 16 + (c & 15) < p.half;
-        else return nt * BN + c < p.N;
-    };
-
     // the chunk's operand pieces: piece i is 16-byte column i % 8 of tile row
     // i / 8 (rows 0..BM-1 tokens, then BN weight rows); rows past the matrix
     // repeat its last row
@@ -347,7 +329,7 @@ __global__ __launch_bounds__(256) void gemm_chain_kernel(GemmParams p) {
             const int i = min((int)threadIdx.x + 256 * q, kPieces - 1);
             const int row = i >> 3, col = i & 7;
             const int8_t* src = row < BM ? p.X + (size_t)min(m0 + row, p.M - 1) * p.K
-                                         : p.W + (size_t)min(weight_row(row - BM), p.N - 1) * p.K;
+                                         : p.W + (size_t)min(nt * BN + row - BM, p.N - 1) * p.K;
             piece[q] = *reinterpret_cast<const v4i*>(src + (size_t)ch * kChunkBytes + 16 * col);
         }
     };
@@ -366,7 +348,7 @@ __global__ __launch_bounds__(256) void gemm_chain_kernel(GemmParams p) {
     const int r16 = lane & 15, kq = lane >> 4;
     int wrow[SN];
 #pragma unroll
-    for (int j = 0; j < SN; ++j) wrow[j] = min(weight_row(wn * SN * 16 + j * 16 + r16), p.N - 1);
+    for (int j = 0; j < SN; ++j) wrow[j] = min(nt * BN + wn * SN * 16 + j * 16 + r16, p.N - 1);
     float4 sw[SN];
     auto load_scales = [&](int ch) {
 #pragma unroll
@@ -446,22 +428,15 @@ __global__ __launch_bounds__(256) void gemm_chain_kernel(GemmParams p) {
         for (int r = 0; r < 4; ++r) {
             const int m = m0 + wm * SM * 16 + i * 16 + 4 * kq + r;
             if (m >= p.M) continue;
-            if constexpr (kSilu) {
-                const int o = nt * (BN / 2) + wn * 16 + r16;
-                if (o < p.half) p.Y[(size_t)m * p.ldy + o] = silu(total[i][0][r]) * total[i][1][r];
-            } else {
 #pragma unroll
-                for (int j = 0; j < SN; ++j) {
-                    const int c = wn * SN * 16 + j * 16 + r16;
-                    if (!row_ok(c)) continue;
-                    float* dst = p.Y + (size_t)m * p.ldy + nt * BN + c;
-                    if constexpr (EPI == kGemmResidual)
-                        *dst = *dst + total[i][j][r];
-                    else if constexpr (EPI == kGemmStoreSilu)
-                        *dst = silu(total[i][j][r]);  // stem.rs:76,99: silu after the stage
-                    else
-                        *dst = total[i][j][r];
-                }
+            for (int j = 0; j < SN; ++j) {
+                const int n = nt * BN + wn * SN * 16 + j * 16 + r16;
+                if (n >= p.N) continue;
+                float* dst = p.Y + (size_t)m * p.ldy + n;
+                if constexpr (EPI == kGemmResidual)
+                    *dst = *dst + total[i][j][r];
+                else
+                    *dst = total[i][j][r];
             }
         }
 }
@@ -737,7 +712,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_ring_kernel(GemmParams p) {
     if ((gridDim.x & 7) == 0) t = (t & 7) * (gridDim.x >> 3) + (t >> 3);  // one weight panel per XCD
     const int mt = t % mtiles, nt = t / mtiles;
     const int m0 = mt * BM, G = p.K / kGroup, chunks = G / 4;
-    auto weight_row = [&](int c) -> int {  // as the chain kernel's
+    auto weight_row = [&](int c) -> int {  // as the panel kernel's
         if constexpr (kSilu) {
             const int w = c / 32, j = (c / 16) & 1, o = nt * (BN / 2) + w * 16 + (c & 15);
             return j == 0 ? o : p.half + o;
@@ -1049,7 +1024,7 @@ static hipError_t launch_product(const GemmParams& p, hipStream_t stream) {
         }
         return launch_chain<1, 1, 2, kGemmRope, FORM, false>(p, stream);
     } else {
-    const int pick = p.K == 1152 ? (EPI == kGemmSilu ? 2 : 3) : chain_pick<EPI>(p);
+    const int pick = p.K == 1152 ? 3 : chain_pick<EPI>(p);
     const int n_eff = EPI == kGemmSilu ? 2 * p.half : p.N;
     const size_t reread = (size_t)((n_eff + 31) / 32) * (size_t)p.M * (size_t)p.K * sizeof(float);
     const bool fused =
@@ -1086,7 +1061,7 @@ hipError_t launch_gemm(const GemmParams& p, int epilogue, int form, bool dump, h
     // instantiated for the supported widths (the kernel is unrolled over groups)
     if ((p.K != 384 && p.K != 512 && p.K != 1024 && p.K != 1152 && p.K != 1536 && p.K != 2048) || p.N <= 0)
         return hipErrorInvalidValue;
-    // 1152 columns (the stem's im2col rows at d 384) have no split-kernel tile: codes only, chain kernel
+    // 1152 columns (the stem's im2col rows at d 384) have no split-kernel tile: codes only, ring kernel
     if (p.K == 1152 && (p.Xf != nullptr || dump)) return hipErrorInvalidValue;
     if (epilogue == kGemmSilu && (p.half % 16 != 0 || p.N != 2 * p.half)) return hipErrorInvalidValue;
     if (epilogue == kGemmRope &&

@@ -666,10 +666,9 @@ struct N3AttendParams {
     int ring_keep, ring_width;
 };
 
-// kernels/src/attention.rs:53-80 for query head blockIdx.x of the token at
-// position + blockIdx.y over positions [first, position + 1) (first from the
-// window, attention.rs:171-177), then times sigmoid(gate)
-// (attention.rs:147-149; attention.rs:319-330 for a run of tokens).
+// kernels/src/attention.rs:53-80 for query head blockIdx.x of one token over
+// positions [first, position + 1) (first from the window, attention.rs:171-177),
+// then times sigmoid(gate) (attention.rs:147-149).
 // Scores are exact; coefficients ((float)score * key_scale) * query_scale; the
 // exponent total is the aarch64 build's: four lane sums over the first
 // count - count % 4 positions (position p in lane p % 4, in order), added as
@@ -681,15 +680,12 @@ __global__ __launch_bounds__(256) void n3_attend_kernel(N3AttendParams p) {
     __shared__ int part[16][kN3Head];
     __shared__ float red[8];
     __shared__ float lanes_s[4];
-    const int t = blockIdx.y, total_positions = p.position + t + 1;
+    const int total_positions = p.position + 1;
     const int first = p.window > 0 && total_positions > p.window ? total_positions - p.window : 0;
-    const int8_t* const qcodes = p.qcodes + (size_t)t * gridDim.x * kN3Head;
-    const float* const gate = p.gate + (size_t)t * p.gate_stride;
-    float* const out = p.out + (size_t)t * gridDim.x * kN3Head;
     const int h = blockIdx.x, tid = threadIdx.x, kvh = h / p.group, count = total_positions - first;
-    const float query_scale = p.qscales[(size_t)t * gridDim.x + h] * p.inverse_root;
+    const float query_scale = p.qscales[h] * p.inverse_root;
     int4 q[4];
-    const int4* qs = reinterpret_cast<const int4*>(qcodes + (size_t)h * kN3Head);
+    const int4* qs = reinterpret_cast<const int4*>(p.qcodes + (size_t)h * kN3Head);
 #pragma unroll
     for (int i = 0; i < 4; ++i) q[i] = qs[i];
     const int8_t* kbase = p.keys + ((size_t)kvh * p.cap + first) * kN3Head;
@@ -751,14 +747,14 @@ __global__ __launch_bounds__(256) void n3_attend_kernel(N3AttendParams p) {
         for (int pp = vector_count; pp < count; ++pp) total = total + c_s[pp];
         float o = cpeak > 0.0f ? (float)sum * scale : 0.0f;
         o = o * reciprocal(total);
-        o = o * libm_sigmoid(gate[(size_t)h * kN3Head + tid]);
-        out[(size_t)h * kN3Head + tid] = o;
+        o = o * libm_sigmoid(p.gate[(size_t)h * kN3Head + tid]);
+        p.out[(size_t)h * kN3Head + tid] = o;
     }
 }
 
-// n3_attend_kernel for a run of `count` tokens on the matrix cores: query head
-// blockIdx.x of the `tile` tokens (a power of two, at most 16) from blockIdx.y *
-// tile, 512 threads, over every position any of them sees. Both contractions are
+// n3_attend_kernel for a run of `count` tokens (attention.rs:319-330) on the matrix
+// cores: query head blockIdx.x of the `tile` tokens (a power of two, at most 16)
+// from blockIdx.y * tile, 512 threads, over every position any of them sees. Both contractions are
 // exact integers, so their order is free: the scores are one
 // v_mfma_i32_16x16x64_i8 per 16 tokens x 16 positions, the 12-bit weights enter as
 // two int8 digits (w = 128 hi + lo) against the value codes, 64 positions an
@@ -1008,25 +1004,18 @@ __global__ __launch_bounds__(kN3TileThreads) void n3_attend_tile_kernel(N3Attend
     }
 }
 
-// ops.rs:120-125 over n <= 4096 values (one block a vector: block b reads in +
-// b * n), then, for group > 0, prepare for a matrix of that group and padded
-// width (matrix.rs:123-128) into out + b * padded (else out + b * n)
+// ops.rs:120-125 over n <= 4096 values of one vector, then prepare for a matrix of
+// that group and padded width (matrix.rs:123-128); one block
 __global__ __launch_bounds__(kN3Block) void n3_fake_quantise_kernel(const float* in, int n, int padded, int group,
                                                                     float wht_scale, float* out) {
     __shared__ float buf[kN3MaxWidth];
     __shared__ float red[32];
-    in += (size_t)blockIdx.x * n;
-    out += (size_t)blockIdx.x * (group > 0 ? padded : n);
     for (int i = threadIdx.x; i < n; i += blockDim.x) buf[i] = in[i];
     __syncthreads();
     n3_fake_quantise(buf, n, red);
-    if (group > 0) {
-        for (int i = n + threadIdx.x; i < padded; i += blockDim.x) buf[i] = 0.0f;
-        __syncthreads();
-        n3_rotate(buf, padded, group, wht_scale);
-    } else {
-        padded = n;
-    }
+    for (int i = n + threadIdx.x; i < padded; i += blockDim.x) buf[i] = 0.0f;
+    __syncthreads();
+    n3_rotate(buf, padded, group, wht_scale);
     for (int i = threadIdx.x; i < padded; i += blockDim.x) out[i] = buf[i];
 }
 
