@@ -137,9 +137,9 @@ constexpr int kNormWindow = 12288;  // bytes of norms staged per row group (3 x 
 // -> rotated [count][padded], zero past `columns`, each group rotated. One
 // lane per run of 16 elements. Bound by latency: a 256 x 768 batch is 192 waves,
 // so a block is one wave (192 CUs load, not 48), a run loads as four 16-byte
-// pieces where rows and base are whole pieces, and the butterflies across lanes are DPP moves
-// instead of LDS permutes: 9.4 -> 4.75 us a launch, 256 x 2048 x 768 (rotation and
-// product, 2 bits) 12.1 -> 9.9 us.
+// pieces where rows and base are whole pieces, and the butterflies across lanes
+// are DPP moves instead of LDS permutes: 9.4 -> 4.7 us a traced launch; a call of
+// rotation and product, 256 x 2048 x 768 of 2 bits, 12.1 -> 9.9 us timed.
 constexpr int kRotateThreads = 64;
 
 template <int GROUP>
@@ -446,9 +446,10 @@ void cb_product_jobs_kernel(CodebookJobs jobs) {
 // A block's quantisation (15 vector operations a value, repeated by every block
 // of a token tile) and the latency of its first loads bound a prompt chunk, the
 // decode and the epilogue (23 vector operations a product at 4 bits) the largest.
-// Measured per call, against tiles of eight tokens on v_dot4: 256 tokens x 2048
-// rows x 768 columns of 2 bits 7.2 us (was 53), 512 x 8192 x 768 18 us (was
-// 330), 4-bit 512 x 8192 x 4096 110 us, 314 TOPS (was 2110).
+// The product timed back to back, against tiles of eight tokens on v_dot4: 256
+// tokens x 2048 rows x 768 columns of 2 bits 6.5 us (was 51; a traced launch, its
+// start and end included, 8.2 and 54), 512 x 8192 x 768 17 us (was 323), 4-bit 512 x
+// 8192 x 4096 109 us, 315 TOPS (was 2110).
 constexpr int kTileWaves = 8;
 constexpr int kTileBatch = 128;                            // bytes of a row per batch
 constexpr int kTileSlot = 16 * (kTileBatch + 16);          // a wave's batch in LDS: rows 16 bytes apart in banks

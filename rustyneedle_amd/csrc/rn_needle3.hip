@@ -1353,7 +1353,8 @@ __global__ __launch_bounds__(256) void n3_observe_kernel(const float* cells, N3O
 // weighted sums' updates (heads.rs:138-155) follow as chains, one a dimension,
 // over cells requested sixteen tokens ahead. One block a slot with the peaks
 // and exponentials token by token in one thread took 153 us for 256 tokens x 84
-// slots x 768 and a launch a head; these take 21 + 32 us for both heads' 168.
+// slots x 768 and a launch a head (traced); these take 21 and 32 us, one pair of
+// launches a chunk for both heads' 168 slots.
 // scores [slot][kN3FeedChunk + 1]: the run's scores, then the peak before it
 // (which the second launch's blocks read while one of them replaces it).
 __device__ __forceinline__ int n3_slot_head(const N3ObserveHeads& hs) {
